@@ -43,6 +43,7 @@ struct Geometry {
   std::array<bool, 2> have_rt{};
   std::array<LegTables, 5> waves;  // base + wave bounds, indexed by RL
   std::array<int64_t, 5> T_exec{};
+  int64_t T_seg = 0;  // of the matrix-core sweeps
   std::array<bool, 5> have{};
 };
 
@@ -56,17 +57,15 @@ struct Shape {
 std::mutex g_wisdom_mu;
 std::map<std::tuple<int, int, int, int>, Shape> g_wisdom;  // (N, L, M, K) -> shape
 
-int heuristic_kb(int K) { return legendre_map_block(K); }
-int heuristic_rl(int K) { return legendre_default_rl(K); }
+int heuristic_kb(const Geometry &g, int K) { return legendre_map_block(K, g.M, 2 * g.N); }
+int heuristic_rl(const Geometry &g, int K) { return legendre_default_rl(K, g.M, 2 * g.N); }
 int heuristic_rw(int K) { return K >= kRingWideMaps ? 1 : 0; }
 
-std::vector<Shape> candidate_shapes(int K) {
+std::vector<Shape> candidate_shapes(const Geometry &g, int K) {
   std::vector<Shape> out;
-  std::vector<int> kbs = {heuristic_kb(K)};
-  if (K > 4) kbs.push_back(8);
-  for (int KB : kbs)
-    for (int RL : {1, 2, 4})
-      if (batch_shape_supported(RL, KB)) out.push_back({RL, KB});
+  const int KB = heuristic_kb(g, K);  // the maps per pass decide the order of the sums
+  for (int RL : {1, 2, 4})
+    if (batch_shape_supported(RL, KB)) out.push_back({RL, KB});
   return out;
 }
 
@@ -155,6 +154,7 @@ Geometry *get_geometry(wavemoth_batch b, int N, int L, int M) {
   g->L = L;
   g->M = M;
   if (!build_leg_geometry(b->arena, g->base, N, L, M, b->stream, &g->cnt)) return nullptr;
+  if (!build_leg_segments(b->arena, g->base, b->stream, &g->T_seg)) return nullptr;
   b->geoms.push_back(std::move(g));
   return b->geoms.back().get();
 }
@@ -393,7 +393,7 @@ double time_rings(wavemoth_batch b, Geometry *g, int K, int w) {
   do {
     if (!ensure_rings(b, g, w)) break;
     LegTables t;
-    if (!request_tables(b->arena, a, g, K, {heuristic_rl(K), heuristic_kb(K), w}, b->stream,
+    if (!request_tables(b->arena, a, g, K, {heuristic_rl(*g, K), heuristic_kb(*g, K), w}, b->stream,
                         &t))
       break;
     if (hipMemsetAsync(t.qbuf, 0, (size_t)q_alloc_elems(t.R, K, t.M + 1) * sizeof(double2),
@@ -444,7 +444,7 @@ bool ring_variants_differ(wavemoth_batch b, Geometry *g, bool *ok) {
 }
 
 bool choose_shape(wavemoth_batch b, Geometry *g, int K, Shape *out, int *measured) {
-  const Shape h = {heuristic_rl(K), heuristic_kb(K), heuristic_rw(K)};
+  const Shape h = {heuristic_rl(*g, K), heuristic_kb(*g, K), heuristic_rw(K)};
   *out = h;
   *measured = 0;
   if (!(b->flags & WAVEMOTH_MEASURE)) return true;
@@ -459,7 +459,7 @@ bool choose_shape(wavemoth_batch b, Geometry *g, int K, Shape *out, int *measure
     }
   }
   double best = -1.0;
-  for (Shape sh : candidate_shapes(K)) {
+  for (Shape sh : candidate_shapes(*g, K)) {
     const double ms = time_shape(b, g, K, sh);
     if (ms < 0) {
       set_err(std::string("autotuner: timing a sweep shape failed: ") + last_err());
@@ -580,7 +580,7 @@ bool build_batch(wavemoth_batch b) {
     if (!request_tables(b->arena, b->arena, g, b->K[r], b->shape[r], b->stream, &b->tabs[r]))
       return false;
     const int nkb = (b->K[r] + b->shape[r].KB - 1) / b->shape[r].KB;
-    b->exec_slots[r] = g->T_exec[b->shape[r].RL] * nkb;
+    b->exec_slots[r] = (legendre_matrix(b->shape[r].KB) ? g->T_seg : g->T_exec[b->shape[r].RL]) * nkb;
     b->sum_eps += g->cnt.T_eps;
     b->sum_dense += g->cnt.T_dense;
     b->sum_flops += (5 + 4 * (int64_t)b->K[r]) * g->cnt.T_eps;

@@ -30,6 +30,9 @@
 
 namespace wm {
 
+// Up to this many maps the sweep's contraction runs on the vector units.
+constexpr int kMapsVector = 3;
+
 // -------------------------------------------------------------- seeds
 
 // One thread per (m, ring).  Writes seed_l / seed_v.
@@ -113,6 +116,54 @@ __global__ __launch_bounds__(256) void k_wave_bounds(LegTables t) {
   t.wseedmax[gid] = hi;
 }
 
+// The first l of each (m, chunk of kSegRings rings) and the recurrence
+// states (L~_{l-1}, L~_l) of its rings at the starts of l-segments 1 .. 3
+// (zero before a ring's seed), with the same steps and chunk rescale as the
+// sweep: ckpt[(3 m + s - 1) R + r].  A segment is ns = ceil(nc / 4) of the nc
+// l-chunks from the first one.  One block per (m, chunk), a thread per ring.
+__global__ __launch_bounds__(kSegRings) void k_checkpoints(LegTables t) {
+  __shared__ int wmin[kSegRings / 64];
+  const int m = blockIdx.x / t.SW, sc = blockIdx.x - m * t.SW;
+  const int r = sc * kSegRings + threadIdx.x, R = t.R, L = t.L;
+  const int sl = r < R ? t.seed_l[(int64_t)m * R + r] : kSeedNone;
+  int lo = sl;
+  for (int d = 32; d >= 1; d >>= 1) {
+    const int o = __shfl_xor(lo, d);
+    lo = o < lo ? o : lo;
+  }
+  if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = lo;
+  __syncthreads();
+  int l0 = wmin[0];
+  for (int i = 1; i < kSegRings / 64; ++i) l0 = wmin[i] < l0 ? wmin[i] : l0;
+  l0 = __builtin_amdgcn_readfirstlane(l0);
+  if (threadIdx.x == 0) t.seg_l0[blockIdx.x] = l0;
+  if (l0 > L) return;
+  const int nc = (L - l0) / kChunk + 1, ns = (nc + 3) / 4;
+  const int64_t offm = t.off[m];
+  const double *ct = t.ctil + (offm - m), *cs = t.cscale + (offm + l0 - m) / kChunk;
+  const double x = r < R ? t.ring_x[r] : 0.0;
+  const double2 sv = sl <= L ? t.seed_v[(int64_t)m * R + r] : make_double2(0.0, 0.0);
+  double prev = 0.0, cur = 0.0;
+  for (int s = 1; s <= 3 && s * ns < nc; ++s) {
+    for (int ch = (s - 1) * ns; ch < s * ns; ++ch) {
+      const int l = l0 + kChunk * ch;
+      if (sl == l) {
+        prev = sv.x;
+        cur = sv.y;
+      }
+#pragma unroll
+      for (int j = 0; j < kChunk; ++j) {
+        const double nx = fma(x, cur, -(ct[l + j] * prev));
+        prev = cur;
+        cur = nx;
+      }
+      prev *= cs[ch];
+      cur *= cs[ch];
+    }
+    if (r < R) t.ckpt[((int64_t)m * 3 + s - 1) * R + r] = make_double2(prev, cur);
+  }
+}
+
 // ------------------------------------------------------- a_lm prescale
 
 // map slots of atil: nmaps rounded up to whole blocks of KB
@@ -168,7 +219,14 @@ __device__ __forceinline__ const WM_CONST T *const_view(const T *p) {
   return (const WM_CONST T *)p;
 }
 
-// The sweep proper.
+// The sweep of up to 3 maps on the vector units: 2 + 2 KB FP64 instructions
+// per (l, ring), their coefficients (c~_l and KB complex a~_l) wave-uniform
+// SGPR operands.  The scalar loads of a step of ST l are issued one step
+// ahead: scalar loads return out of order, so a wait for one is a wait for
+// all, and a step that loads what it uses itself stalls for the whole L2
+// latency.  The empty asm marks where the step's own values must have
+// arrived; the next step's loads follow it and have the step's arithmetic
+// (ST RL (2 + 2 KB) instructions) to arrive.
 template <int RL, int KB>
 __device__ __forceinline__ void legendre_sweep(
     int L, int R, int Mp1, int K, int m, int w, int kbase, int lane, int l0, int lsmax,
@@ -176,7 +234,9 @@ __device__ __forceinline__ void legendre_sweep(
     const WM_CONST double *cs, const double *__restrict__ ring_x,
     const int *__restrict__ seed_l, const double2 *__restrict__ seed_v,
     double2 *__restrict__ qbuf) {
+  constexpr int ST = KB <= 2 ? 4 : 2;  // l per step: both steps' values fit the SGPRs
   double x[RL], prev[RL], cur[RL];
+  double2 sv[RL];
   int sl[RL], rr[RL];
   double acc[RL][2][KB][2];
 #pragma unroll
@@ -185,6 +245,7 @@ __device__ __forceinline__ void legendre_sweep(
     const bool ok = rr[i] < R;
     x[i] = ok ? ring_x[rr[i]] : 0.0;
     sl[i] = ok ? seed_l[(int64_t)m * R + rr[i]] : kSeedNone;
+    sv[i] = ok ? seed_v[(int64_t)m * R + rr[i]] : make_double2(0.0, 0.0);
     prev[i] = 0.0;
     cur[i] = 0.0;
 #pragma unroll
@@ -193,53 +254,65 @@ __device__ __forceinline__ void legendre_sweep(
       for (int k = 0; k < KB; ++k) acc[i][p][k][0] = acc[i][p][k][1] = 0.0;
   }
 
-  for (; l0 <= L; l0 += kChunk) {
-    if (l0 <= lsmax) {
+  if (l0 <= L) {
+    double c[ST], a[ST][2 * KB], S;
+    const int last = m + (L - m) / kChunk * kChunk + kChunk - ST;  // start of the last step
 #pragma unroll
-      for (int i = 0; i < RL; ++i) {
-        if (sl[i] == l0) {
-          const double2 v = seed_v[(int64_t)m * R + rr[i]];
-          prev[i] = v.x;
-          cur[i] = v.y;
-        }
-      }
+    for (int j = 0; j < ST; ++j) {
+      c[j] = ct[l0 + j];
+#pragma unroll
+      for (int u = 0; u < 2 * KB; ++u) a[j][u] = at[2 * (int64_t)KB * (l0 + j) + u];
     }
+    S = cs[(l0 - m) / kChunk];
+    for (; l0 <= L; l0 += kChunk) {
+      if (l0 <= lsmax) {
 #pragma unroll
-    for (int j = 0; j < kChunk; j += 2) {
-      const int l = l0 + j;
-      const double c0 = ct[l], c1 = ct[l + 1];
-      double2 a0[KB], a1[KB];
-#pragma unroll
-      for (int k = 0; k < KB; ++k) {
-        const int64_t i0 = 2 * ((int64_t)l * KB + k), i1 = i0 + 2 * KB;
-        a0[k] = make_double2(at[i0], at[i0 + 1]);
-        a1[k] = make_double2(at[i1], at[i1 + 1]);
-      }
-#pragma unroll
-      for (int i = 0; i < RL; ++i) {
-#pragma unroll
-        for (int k = 0; k < KB; ++k) {
-          acc[i][0][k][0] = fma(cur[i], a0[k].x, acc[i][0][k][0]);
-          acc[i][0][k][1] = fma(cur[i], a0[k].y, acc[i][0][k][1]);
+        for (int i = 0; i < RL; ++i) {
+          prev[i] = sl[i] == l0 ? sv[i].x : prev[i];
+          cur[i] = sl[i] == l0 ? sv[i].y : cur[i];
         }
-        const double n1 = fma(x[i], cur[i], -(c0 * prev[i]));
-        prev[i] = cur[i];
-        cur[i] = n1;
-#pragma unroll
-        for (int k = 0; k < KB; ++k) {
-          acc[i][1][k][0] = fma(cur[i], a1[k].x, acc[i][1][k][0]);
-          acc[i][1][k][1] = fma(cur[i], a1[k].y, acc[i][1][k][1]);
-        }
-        const double n2 = fma(x[i], cur[i], -(c1 * prev[i]));
-        prev[i] = cur[i];
-        cur[i] = n2;
       }
-    }
-    const double S = cs[(l0 - m) / kChunk];
+      double Sn = S;
 #pragma unroll
-    for (int i = 0; i < RL; ++i) {
-      prev[i] *= S;
-      cur[i] *= S;
+      for (int j0 = 0; j0 < kChunk; j0 += ST) {
+        const int ln = l0 + j0 < last ? l0 + j0 + ST : last;
+        asm volatile("" ::"s"(a[ST - 1][2 * KB - 1]), "s"(c[ST - 1]), "s"(S));
+        __builtin_amdgcn_sched_barrier(0);
+        double cn[ST], an[ST][2 * KB];
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+          cn[j] = ct[ln + j];
+#pragma unroll
+          for (int u = 0; u < 2 * KB; ++u) an[j][u] = at[2 * (int64_t)KB * (ln + j) + u];
+        }
+        if (j0 == kChunk - ST) Sn = cs[(ln - m) / kChunk];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < RL; ++i) {
+#pragma unroll
+          for (int j = 0; j < ST; ++j) {
+#pragma unroll
+            for (int k = 0; k < KB; ++k) {
+              acc[i][j & 1][k][0] = fma(cur[i], a[j][2 * k], acc[i][j & 1][k][0]);
+              acc[i][j & 1][k][1] = fma(cur[i], a[j][2 * k + 1], acc[i][j & 1][k][1]);
+            }
+            const double nx = fma(x[i], cur[i], -(c[j] * prev[i]));
+            prev[i] = cur[i];
+            cur[i] = nx;
+          }
+          if (j0 == kChunk - ST) {
+            prev[i] *= S;
+            cur[i] *= S;
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+          c[j] = cn[j];
+#pragma unroll
+          for (int u = 0; u < 2 * KB; ++u) a[j][u] = an[j][u];
+        }
+      }
+      S = Sn;
     }
   }
 
@@ -258,37 +331,219 @@ __device__ __forceinline__ void legendre_sweep(
   }
 }
 
+typedef double leg_d4 __attribute__((ext_vector_type(4)));
+
+// The sweep of KB maps (even, 2 .. 16) with the contraction on the FP64
+// matrix cores.  The chunk's l-range is cut into four segments and the four
+// 16-lane rows of the wave step one segment each, all for the same rings:
+// lane 16 g + i holds Lambda_{l_g}(ring 16 j + i), l_g = step s of segment g,
+// which is the A operand of a product of 16 rings x 4 l as it stands
+// (a product only needs A and B to agree on the l of each k).  Columns are
+// the real and imaginary parts of the pass's maps: v_mfma_f64_16x16x4f64 for
+// every 8 maps, v_mfma_f64_4x4x4f64 (4 blocks of 4 rings, the same 4 columns)
+// for every further 2.  Segments 1 .. 3 start from checkpoints of the
+// recurrence (k_checkpoints), made once per geometry.
+//
+// Why so: an FP64 matrix instruction keeps its SIMD's whole vector unit busy
+// (measured: any vector instruction of another wave adds to its time), so
+// the time is the sum 4 RL (2 + 2) FP64 instructions of the recurrence and
+// 4 RL KB / 2 quarter products per step, and nothing may be added to it.  A
+// wave that steps one l-range per lane has to transpose Lambda first: 16
+// lane swaps per 8 l and 64 rings (8.5 cycles each, +30 % at 16 maps) or an
+// LDS round trip (LDS-bound below 8 maps).  The coefficients and the a~ rows
+// differ by segment and come by vector loads, four steps ahead; in order,
+// unlike scalar loads.
+template <int RL, int KB>
+__device__ __forceinline__ void legendre_sweep_mm(
+    int L, int R, int Mp1, int K, int m, int w, int kbase, int lane, int l0,
+    const double *__restrict__ ct, const double *__restrict__ at,
+    const double *__restrict__ cs, const double *__restrict__ ring_x,
+    const int *__restrict__ seed_l, const double2 *__restrict__ seed_v,
+    const double2 *__restrict__ ckpt, double2 *__restrict__ qbuf) {
+  constexpr int GR = 4 * RL;                      // 16-ring groups
+  constexpr int C16 = KB / 8, C4 = (KB % 8) / 2;  // 16-column tiles, 4-column groups
+  constexpr int B16 = C16 > 0 ? C16 : 1, B4 = C4 > 0 ? C4 : 1;
+  constexpr int ST = KB <= 6 ? 4 : 2;             // steps per load block
+  const int kq = lane >> 4, col = lane & 15, rbase = w * 64 * RL + col;
+  double x[GR], prev[GR], cur[GR];
+  int sl[GR];
+  leg_d4 acc16[GR][2][B16];
+  double acc4[GR][2][B4];
+#pragma unroll
+  for (int i = 0; i < GR; ++i)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+      for (int c = 0; c < B16; ++c) acc16[i][p][c] = leg_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int c = 0; c < B4; ++c) acc4[i][p][c] = 0.0;
+    }
+
+  if (l0 <= L) {
+    const int nc = (L - l0) / kChunk + 1, ns = (nc + 3) / 4;  // chunks, chunks per segment
+    const int cb = kq * ns;                                   // the lane's first chunk
+#pragma unroll
+    for (int i = 0; i < GR; ++i) {
+      const int r = rbase + 16 * i;
+      const bool ok = r < R;
+      x[i] = ok ? ring_x[r] : 0.0;
+      sl[i] = ok ? seed_l[(int64_t)m * R + r] : kSeedNone;
+      double2 v = make_double2(0.0, 0.0);
+      if (ok && kq > 0 && cb < nc) v = ckpt[((int64_t)m * 3 + kq - 1) * R + r];
+      prev[i] = v.x;
+      cur[i] = v.y;
+    }
+    ct += l0;
+    at += 2 * (int64_t)KB * l0;
+    cs += (l0 - m) / kChunk;
+    // row e of the lane's segment: c~ at ct[e], a~ at at[2 KB e + column]
+    unsigned e = kChunk * (unsigned)(cb < nc ? cb : nc - 1);
+    double c[ST], S, b16[ST][B16], b4[ST][B4];
+    auto load = [&](unsigned el, double (&cc)[ST], double (&v16)[ST][B16], double (&v4)[ST][B4]) {
+      const unsigned o16 = 2 * KB * el + col, o4 = 2 * KB * el + 16 * C16 + (lane & 3);
+#pragma unroll
+      for (int j = 0; j < ST; ++j) {
+        cc[j] = ct[el + j];
+#pragma unroll
+        for (int u = 0; u < C16; ++u) v16[j][u] = at[o16 + 2 * KB * j + 16 * u];
+#pragma unroll
+        for (int u = 0; u < C4; ++u) v4[j][u] = at[o4 + 2 * KB * j + 4 * u];
+      }
+    };
+    load(e, c, b16, b4);
+    S = cs[e / kChunk];
+    for (int j = 0; j < ns; ++j) {
+      const int ls = l0 + kChunk * (cb + j);
+      bool hit = false;
+#pragma unroll
+      for (int i = 0; i < GR; ++i) hit |= sl[i] == ls;
+      if (__any(hit)) {
+#pragma unroll
+        for (int i = 0; i < GR; ++i)
+          if (sl[i] == ls) {
+            const double2 v = seed_v[(int64_t)m * R + rbase + 16 * i];
+            prev[i] = v.x;
+            cur[i] = v.y;
+          }
+      }
+      if (3 * ns + j >= nc && cb + j >= nc) {  // past the segment's rows
+#pragma unroll
+        for (int i = 0; i < GR; ++i) prev[i] = cur[i] = 0.0;
+      }
+      const unsigned en = kChunk * (unsigned)(cb + j + 1 < nc ? cb + j + 1 : nc - 1);
+      double Sn = S;
+#pragma unroll
+      for (int s0 = 0; s0 < kChunk; s0 += ST) {
+        double cn[ST], bn16[ST][B16], bn4[ST][B4];
+        load(s0 + ST < kChunk ? e + s0 + ST : en, cn, bn16, bn4);
+        if (s0 + ST == kChunk) Sn = cs[en / kChunk];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < ST; ++s)
+#pragma unroll
+          for (int i = 0; i < GR; ++i) {
+#pragma unroll
+            for (int u = 0; u < C16; ++u)
+              acc16[i][s & 1][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                  cur[i], b16[s][u], acc16[i][s & 1][u], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < C4; ++u)
+              acc4[i][s & 1][u] = __builtin_amdgcn_mfma_f64_4x4x4f64(
+                  cur[i], b4[s][u], acc4[i][s & 1][u], 0, 0, 0);
+            const double nx = fma(x[i], cur[i], -(c[s] * prev[i]));
+            prev[i] = cur[i];
+            cur[i] = nx;
+          }
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+          c[s] = cn[s];
+#pragma unroll
+          for (int u = 0; u < C16; ++u) b16[s][u] = bn16[s][u];
+#pragma unroll
+          for (int u = 0; u < C4; ++u) b4[s][u] = bn4[s][u];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < GR; ++i) {
+        prev[i] *= S;
+        cur[i] *= S;
+      }
+      S = Sn;
+      e = en;
+    }
+  }
+
+  // D of a 16-column tile: ring 16 i + kq + 4 j in register j, column col; of
+  // a 4-column group: ring 16 i + 4 (col / 4) + kq, column col % 4.  Rows of
+  // q (ring, parity) are `row` doubles apart.
+  const int G = q_group(K);
+  const int64_t row = 2 * (int64_t)q_groups(K) * Mp1 * G;
+#pragma unroll
+  for (int u = 0; u < C16 + C4; ++u) {
+    const bool wide = u < C16;
+    const int k = kbase + (wide ? 8 * u + (col >> 1) : 8 * C16 + 2 * (u - C16) + ((col & 3) >> 1));
+    const int rl = w * 64 * RL + kq + (wide ? 0 : (col & 12));  // the lane's first ring
+    if (k >= K) continue;
+    double *q = (double *)qbuf + 2 * q_index(rl, 0, k, m, K, Mp1) + (col & 1);
+#pragma unroll
+    for (int i = 0; i < GR; ++i) {
+      const int ro = 16 * i;
+      if (wide) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (rl + ro + 4 * j < R) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+              q[(2 * (ro + 4 * j) + p) * row] = acc16[i][p][wide ? u : 0][j];
+          }
+      } else if (rl + ro < R) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) q[(2 * ro + p) * row] = acc4[i][p][wide ? 0 : u - C16];
+      }
+    }
+  }
+}
+
 // One wave's share of the sweep: ring chunk w (rings w*64*RL + lane + 64*i,
 // i < RL) of m, maps kb*KB .. kb*KB+KB-1.  Used by the grid kernel below
 // and by the batched work-queue kernel.
 template <int RL, int KB>
 __device__ __forceinline__ void legendre_item(const LegTables &t, int m, int w, int kb,
                                               int lane) {
-  const int l0 = __builtin_amdgcn_readfirstlane(t.wstart[(int64_t)m * t.W + w]);
-  const int lsmax = __builtin_amdgcn_readfirstlane(t.wseedmax[(int64_t)m * t.W + w]);
   const int64_t offm = t.off[m];
-  legendre_sweep<RL, KB>(
-      t.L, t.R, t.M + 1, t.K, m, w, kb * KB, lane, l0, lsmax, const_view(t.ctil + (offm - m)),
-      const_view((const double *)(t.atil + ((int64_t)kb * t.nlpad + offm - m) * KB)),
-      const_view(t.cscale + offm / kChunk), t.ring_x, t.seed_l, t.seed_v, t.qbuf);
+  const double *at = (const double *)(t.atil + ((int64_t)kb * t.nlpad + offm - m) * KB);
+  if constexpr (KB <= kMapsVector) {
+    const int l0 = __builtin_amdgcn_readfirstlane(t.wstart[(int64_t)m * t.W + w]);
+    const int lsmax = __builtin_amdgcn_readfirstlane(t.wseedmax[(int64_t)m * t.W + w]);
+    legendre_sweep<RL, KB>(t.L, t.R, t.M + 1, t.K, m, w, kb * KB, lane, l0, lsmax,
+                           const_view(t.ctil + (offm - m)), const_view(at),
+                           const_view(t.cscale + offm / kChunk), t.ring_x, t.seed_l, t.seed_v,
+                           t.qbuf);
+  } else {
+    const int sc = w * RL * 64 / kSegRings;
+    const int l0 = __builtin_amdgcn_readfirstlane(t.seg_l0[(int64_t)m * t.SW + sc]);
+    legendre_sweep_mm<RL, KB>(t.L, t.R, t.M + 1, t.K, m, w, kb * KB, lane, l0,
+                              t.ctil + (offm - m), at, t.cscale + offm / kChunk, t.ring_x,
+                              t.seed_l, t.seed_v, t.ckpt, t.qbuf);
+  }
 }
 
-// Block = 4 waves.  Block b runs on XCD b % 8; every m's blocks are kept
-// on one XCD (m = xcd + 8 * i) so the per-m coefficient rows are fetched
-// into one L2 only, and each XCD walks its m's from cheap-to-start (small
-// m, long l-range) to short ones.
+// One wave per block: waves of one m run for different times (a ring near
+// the pole joins late or never), and a block's slots are only refilled
+// together.  Block b runs on XCD b % 8; every m's blocks are kept on one XCD
+// (m = xcd + 8 * i) so the per-m coefficient rows are fetched into one L2
+// only, and each XCD walks its m's from cheap-to-start (small m, long
+// l-range) to short ones, within an m from the equator to the pole, the map
+// blocks of a ring chunk side by side.
 template <int RL, int KB>
-__global__ __launch_bounds__(256) void k_legendre(LegTables t, int nkb, int bpm) {
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
+__global__ __launch_bounds__(64) void k_legendre(LegTables t, int nkb, int bpm) {
   const int b = blockIdx.x;
   const int s = b >> 3;
   const int m = (b & 7) + 8 * (s / bpm);
   if (m > t.M) return;
-  const int item = (s % bpm) * 4 + wv;
-  if (item >= t.W * nkb) return;
-  const int kb = item / t.W, w = item - kb * t.W;
-  legendre_item<RL, KB>(t, m, w, kb, lane);
+  const int item = s % bpm;
+  const int w = item / nkb, kb = item - w * nkb;
+  legendre_item<RL, KB>(t, m, w, kb, threadIdx.x);
 }
 
 // ------------------------------------------------------------ launchers
@@ -301,23 +556,47 @@ hipError_t launch_seeds(const LegTables &t, hipStream_t s) {
   return hipGetLastError();
 }
 
+hipError_t launch_checkpoints(const LegTables &t, hipStream_t s) {
+  hipLaunchKernelGGL(k_checkpoints, dim3((unsigned)((t.M + 1) * t.SW)), dim3(kSegRings), 0, s, t);
+  return hipGetLastError();
+}
+
 hipError_t launch_wave_bounds(const LegTables &t, hipStream_t s) {
   const int64_t n = (int64_t)(t.M + 1) * t.W;
   hipLaunchKernelGGL(k_wave_bounds, dim3(nblocks(n, 256)), dim3(256), 0, s, t);
   return hipGetLastError();
 }
 
-// Maps per pass (KB) from nmaps; rings per lane (RL) is a plan choice
-// (heuristic below, or measured by the autotuner).  Two rings per lane and
-// at most four maps a pass: each wave then reads a coefficient row for
-// twice the rings, and the 8-map pass's registers (3 waves per SIMD at two
-// rings) are avoided; measured at Nside 2048, lmax 4096, the sweep takes
-// 140 ms at 64 maps against 222 ms with one ring and 8 maps per pass
-// (18.3 against 27.9 at 8 maps, 7.8 against 11.9 at 3).
-int legendre_map_block(int K) { return K <= 4 ? K : 4; }
-int legendre_default_rl(int K) { return 2; }
-int legendre_padded_maps(int K) {
-  const int KB = legendre_map_block(K);
+// Maps per pass (KB) of the sweep: up to kMapsVector maps in one pass on the
+// vector units, more in passes of at most 16 on the matrix cores, all of one
+// even size.  Measured, ms of one sweep at lmax = 2 Nside = 2048 (vector with
+// four maps a pass / vector of this form / matrix cores): 1 map 0.64 / 0.60 /
+// 1.35, 2 maps 0.91 / 0.81 / 0.95, 3 maps 1.24 / 1.23 / 1.40, 4 maps 1.53 / - /
+// 1.40, 6 maps 2.97 / - / 1.87, 8 maps 2.92 / - / 2.02, 64 maps 23.2 / - / 14.2.
+// Geometries of few waves are bound by the length of a wave, not by the
+// chip's rate; the matrix form's four segments make it four times shorter.
+// Waves of the vector form at which the two are even: 3 maps between 3072
+// (Nside 256, lmax 767: 114 / 79 us) and 8200 (Nside 512: 207 / 250 us),
+// fewer maps between 514 (Nside 128: 23 / 17 us) and 2052 (Nside 256: 44 / 45).
+int legendre_map_block(int K, int M, int R) {
+  if (K <= kMapsVector) {
+    const int64_t waves = (int64_t)(M + 1) * ((R + 127) / 128);
+    return waves < (K < 3 ? 1024 : 6144) ? kMapsVector + 1 : K;
+  }
+  const int passes = (K + 15) / 16, kb = (K + passes - 1) / passes;
+  return (kb + 1) / 2 * 2;
+}
+bool legendre_matrix(int KB) { return KB > kMapsVector; }
+// Rings per wave / 64: two on the vector units (each coefficient row then
+// serves twice the rings; one: 0.87 ms where two take 0.60), two on the matrix
+// cores while the accumulators leave two waves per SIMD and the waves fill
+// the chip (6 maps: 1.87 ms, with one 2.01; 8 maps: 2.08, with one 2.02).
+int legendre_default_rl(int K, int M, int R) {
+  const int KB = legendre_map_block(K, M, R);
+  if (!legendre_matrix(KB)) return 2;
+  return KB <= 6 && (int64_t)(M + 1) * ((R + 127) / 128) >= 2048 ? 2 : 1;
+}
+int legendre_padded_maps(int K, int KB) {
   return ((K + KB - 1) / KB) * KB;
 }
 
@@ -333,22 +612,11 @@ hipError_t launch_prep_alm(const LegTables &t, const double2 *alm, hipStream_t s
 template <int RL, int KB>
 static hipError_t launch_leg_t(const LegTables &t, hipStream_t s) {
   const int nkb = (t.K + KB - 1) / KB;
-  const int bpm = (t.W * nkb + 3) / 4;
+  const int bpm = t.W * nkb;
   const int mgroups = (t.M + 1 + 7) / 8;
   const unsigned grid = (unsigned)(8 * mgroups * bpm);
-  hipLaunchKernelGGL((k_legendre<RL, KB>), dim3(grid), dim3(256), 0, s, t, nkb, bpm);
+  hipLaunchKernelGGL((k_legendre<RL, KB>), dim3(grid), dim3(64), 0, s, t, nkb, bpm);
   return hipGetLastError();
-}
-
-template <int RL>
-static hipError_t launch_leg_rl(const LegTables &t, hipStream_t s) {
-  switch (t.KB) {
-    case 1: return launch_leg_t<RL, 1>(t, s);
-    case 2: return launch_leg_t<RL, 2>(t, s);
-    case 3: return launch_leg_t<RL, 3>(t, s);
-    case 4: return launch_leg_t<RL, 4>(t, s);
-    default: return launch_leg_t<RL, 8>(t, s);
-  }
 }
 
 // ---------------------------------------------------------------- batch
@@ -383,8 +651,11 @@ __global__ __launch_bounds__(256) void k_batch_prep(BatchDev b) {
   prep_entry(t, b.alm[lo], j, (int)(u - j * Kp), t.KB);
 }
 
-#define WM_BATCH_SHAPES(X) \
-  X(1, 1) X(1, 2) X(1, 3) X(1, 4) X(1, 8) X(2, 1) X(2, 2) X(2, 3) X(2, 4) X(2, 8) X(4, 1)
+// (RL, KB) shapes of the sweep
+#define WM_SWEEP_SHAPES(X)                                                    \
+  X(1, 1) X(1, 2) X(1, 3) X(2, 1) X(2, 2) X(2, 3) X(4, 1) X(4, 2) X(4, 3)     \
+  X(1, 4) X(2, 4) X(1, 6) X(2, 6) X(1, 8) X(2, 8)                             \
+  X(1, 10) X(1, 12) X(1, 14) X(1, 16)
 
 bool batch_shape_supported(int RL, int KB) { return batch_shape_index(RL, KB) >= 0; }
 
@@ -393,7 +664,7 @@ int batch_shape_index(int RL, int KB) {
 #define WM_IDX(R_, K_)                     \
   if (RL == R_ && KB == K_) return i;      \
   ++i;
-  WM_BATCH_SHAPES(WM_IDX)
+  WM_SWEEP_SHAPES(WM_IDX)
 #undef WM_IDX
   return -1;
 }
@@ -429,6 +700,9 @@ __global__ __launch_bounds__(256) void k_batch_legendre(BatchDev b, int first, i
     t.seed_v = tp->seed_v;
     t.wstart = tp->wstart;
     t.wseedmax = tp->wseedmax;
+    t.SW = tp->SW;
+    t.seg_l0 = tp->seg_l0;
+    t.ckpt = tp->ckpt;
     t.atil = tp->atil;
     t.qbuf = tp->qbuf;
     legendre_item<R_, K_>(t, m, w, kb, lane);
@@ -451,7 +725,7 @@ hipError_t batch_legendre_occupancy(int RL, int KB, int *blocks_per_cu) {
   if (RL == R_ && KB == K_)                                                              \
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu,                   \
                                                         k_batch_legendre<R_, K_>, 256, 0);
-  WM_BATCH_SHAPES(WM_OCC)
+  WM_SWEEP_SHAPES(WM_OCC)
 #undef WM_OCC
   return hipErrorInvalidValue;
 }
@@ -465,18 +739,17 @@ hipError_t launch_batch_legendre(const BatchDev &b, int RL, int KB, int first, i
                        count, ctr);                                                      \
     return hipGetLastError();                                                            \
   }
-  WM_BATCH_SHAPES(WM_LAUNCH)
+  WM_SWEEP_SHAPES(WM_LAUNCH)
 #undef WM_LAUNCH
   return hipErrorInvalidValue;
 }
 
 hipError_t launch_legendre(const LegTables &t, hipStream_t s) {
-  switch (t.RL) {
-    case 1: return launch_leg_rl<1>(t, s);
-    case 2: return launch_leg_rl<2>(t, s);
-    case 4: return launch_leg_rl<4>(t, s);
-    default: return hipErrorInvalidValue;
-  }
+#define WM_LAUNCH(R_, K_) \
+  if (t.RL == R_ && t.KB == K_) return launch_leg_t<R_, K_>(t, s);
+  WM_SWEEP_SHAPES(WM_LAUNCH)
+#undef WM_LAUNCH
+  return hipErrorInvalidValue;
 }
 
 }  // namespace wm

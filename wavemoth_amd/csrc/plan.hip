@@ -250,16 +250,39 @@ bool build_leg_waves(DevArena &a, LegTables &t, int RL, hipStream_t stream, int6
   return true;
 }
 
+bool build_leg_segments(DevArena &a, LegTables &t, hipStream_t stream, int64_t *T_exec) {
+  t.SW = (t.R + kSegRings - 1) / kSegRings;
+  if (!dalloc(a, &t.seg_l0, (size_t)(t.M + 1) * t.SW, "segment starts")) return false;
+  if (!dalloc(a, &t.ckpt, (size_t)(t.M + 1) * 3 * t.R, "recurrence checkpoints")) return false;
+  WM_TRY(launch_checkpoints(t, stream), "checkpoint kernel");
+  std::vector<int> l0((size_t)(t.M + 1) * t.SW);
+  WM_TRY(hipMemcpyAsync(l0.data(), t.seg_l0, l0.size() * sizeof(int), hipMemcpyDeviceToHost,
+                        stream),
+         "segment starts download");
+  WM_TRY(hipStreamSynchronize(stream), "checkpoint kernel");
+  int64_t tx = 0;
+  for (int v : l0)
+    if (v <= t.L) {
+      const int64_t nc = (t.L - v) / kChunk + 1;
+      tx += (nc + 3) / 4 * 4 * kChunk * kSegRings;
+    }
+  *T_exec = tx;
+  return true;
+}
+
 }  // namespace wm
 
 static bool build_legendre_tables(wavemoth_plan p) {
   LegTables &t = p->lt;
   if (!build_leg_geometry(p->arena, t, p->N, p->L, p->M, p->stream, &p->cnt)) return false;
-  int RL = p->rl_choice > 0 ? p->rl_choice : legendre_default_rl(p->K);
+  int RL = p->rl_choice > 0 ? p->rl_choice : legendre_default_rl(p->K, t.M, t.R);
   if (p->mix >= 0) RL = mix_rings_per_lane_table();  // one wave-table entry per workgroup
+  int64_t T_seg = 0;
+  if (!build_leg_segments(p->arena, t, p->stream, &T_seg)) return false;
   if (!build_leg_waves(p->arena, t, RL, p->stream, &p->T_exec)) return false;
   t.K = p->K;
-  t.KB = legendre_map_block(p->K);
+  t.KB = legendre_map_block(p->K, t.M, t.R);
+  if (p->mix < 0 && legendre_matrix(t.KB)) p->T_exec = T_seg;
   if (p->mix >= 0) {
     // the mixed path reads the pre-split B operand instead of atil
     const int cpb = mix_cols_per_block();
@@ -329,7 +352,7 @@ static bool build_legendre_tables(wavemoth_plan p) {
       WM_TRY(hipStreamSynchronize(p->stream), "checkpoint kernel");
     }
     if (!dalloc(p->arena, &t.atil, 1, "atil")) return false;
-  } else if (!dalloc(p->arena, &t.atil, (size_t)t.nlpad * legendre_padded_maps(p->K), "atil")) {
+  } else if (!dalloc(p->arena, &t.atil, (size_t)t.nlpad * legendre_padded_maps(p->K, t.KB), "atil")) {
     return false;
   }
   // mixed-precision plans store q in FP32 (float2 elements at the same
@@ -712,6 +735,7 @@ static bool run_legendre(wavemoth_plan p, const double2 *d_alm, hipStream_t s) {
   if (p->fly) {
     WM_TRY(launch_seeds(p->lt, s), "seed kernel");
     WM_TRY(launch_wave_bounds(p->lt, s), "wave-bounds kernel");
+    WM_TRY(launch_checkpoints(p->lt, s), "checkpoint kernel");
     if (p->mix_ckpt)
       WM_TRY(launch_mix_ckpt(p->lt, p->mix_dtil, p->mix_etil, p->mix_gtil, p->mix_lam_scale,
                              p->mix_ckpt, s),

@@ -79,6 +79,10 @@ bool build_leg_geometry(DevArena &a, LegTables &t, int N, int L, int M, hipStrea
 // the number of (l, ring) slots the sweep executes with them.
 bool build_leg_waves(DevArena &a, LegTables &t, int RL, hipStream_t s, int64_t *T_exec);
 
+// l-segments of the matrix-core sweeps (t.SW, t.seg_l0, t.ckpt, from the
+// seeds) and the (l, ring) slots such a sweep executes.
+bool build_leg_segments(DevArena &a, LegTables &t, hipStream_t s, int64_t *T_exec);
+
 // Rings of the long path (kRingLong), in groups of one transform length P
 // (P = h for a power-of-two h, else the Bluestein length): entries
 // vecs[first .. first + count) of (ring pair, hemisphere); with K maps a

@@ -17,6 +17,8 @@ constexpr int kChunk = 16;
 // seed_l value of a (m, ring) column whose |Lambda| never reaches the
 // start threshold for l <= lmax.
 constexpr int kSeedNone = 0x3fffffff;
+// Rings that share their l-segments (LegTables::seg_l0).
+constexpr int kSegRings = 128;
 // Largest power-of-two FFT length held in LDS by the ring kernels
 // (8192 complex doubles = 128 KiB).
 constexpr int kMaxFFT = 8192;
@@ -33,7 +35,7 @@ constexpr int kRingThreads = 512;
 // Device tables of the Legendre stage, all owned by one plan.
 struct LegTables {
   int N = 0, L = 0, M = 0, K = 0, R = 0;
-  int RL = 0;        // rings per lane
+  int RL = 0;        // rings per wave / 64
   int KB = 0;        // maps per sweep pass (atil holds ceil(K/KB)*KB maps)
   int W = 0;         // ring chunks (waves) per m
   int64_t nlpad = 0; // padded l entries over all m
@@ -49,6 +51,10 @@ struct LegTables {
   double2 *seed_v = nullptr;  // [(M+1)*R] (Lambda_{l-1} a_{l-1}, Lambda_l)
   int *wstart = nullptr;      // [(M+1)*W] min seed_l over a wave's rings
   int *wseedmax = nullptr;    // [(M+1)*W] max seed_l (<= lmax) over a wave
+  // l-segments of the matrix-core sweeps (k_checkpoints), null without them
+  int SW = 0;                 // chunks of kSegRings rings
+  int *seg_l0 = nullptr;      // [(M+1)*SW] min seed_l over a chunk's rings
+  double2 *ckpt = nullptr;    // [(M+1)*3*R] states at the starts of segments 1 .. 3
   double2 *atil = nullptr;    // [ceil(K/KB)][nlpad][KB] prescaled a_lm (per execute)
   double2 *qbuf = nullptr;    // [R][2][K][M+1] even/odd Legendre sums (q_index)
   int q32 = 0;                // q stored as float2 at the same indices (mixed plans)
@@ -157,7 +163,7 @@ struct BatchRing16Item {
 };
 // queue heads of the sweep shapes (one persistent kernel per shape)
 constexpr int kBatchCounters = 64;
-constexpr int kBatchSweepCtr = 48;  // queue head of sweep shape i: kBatchSweepCtr + i
+constexpr int kBatchSweepCtr = 32;  // queue head of sweep shape i: kBatchSweepCtr + i
 struct BatchDev {
   int nreq = 0;
   const LegTables *tabs = nullptr;      // [nreq] per-request tables (K, KB, RL, buffers)
@@ -228,10 +234,12 @@ hipError_t launch_mixr(const LegTables &t, const void *bmat, int NCp, int64_t pa
                        const double *btab, const double *gtab, const double2 *ckpt,
                        hipStream_t s);
 
-// Shape of the Legendre sweep for nmaps = K.
-int legendre_map_block(int K);
-int legendre_default_rl(int K);
-int legendre_padded_maps(int K);
+// Shape of the Legendre sweep for nmaps = K on a geometry: maps per pass KB,
+// rings per wave / 64; whether the passes run on the matrix cores; map slots.
+int legendre_map_block(int K, int M, int R);
+int legendre_default_rl(int K, int M, int R);
+bool legendre_matrix(int KB);
+int legendre_padded_maps(int K, int KB);
 
 // One strip of a resource matrix on the device (the Legendre stage read
 // from a rev1 file): rows `row`.. of (m, odd) (l = m + odd + 2 row), nks of
@@ -277,6 +285,7 @@ hipError_t launch_res_interp(const LegTables &t, const double *img, const ResInt
 // Launchers (return hipError_t of the launch).
 hipError_t launch_seeds(const LegTables &t, hipStream_t s);
 hipError_t launch_wave_bounds(const LegTables &t, hipStream_t s);
+hipError_t launch_checkpoints(const LegTables &t, hipStream_t s);
 hipError_t launch_prep_alm(const LegTables &t, const double2 *alm, hipStream_t s);
 hipError_t launch_legendre(const LegTables &t, hipStream_t s);
 // Bluestein tables of the lengths hlist[0..nh): chirp[choff + a] =
