@@ -17,8 +17,8 @@
 //     bins past n/2), then q_even = F_north + F_south, q_odd = F_north -
 //     F_south (the equator ring feeds both), into the [R][2][M+1][K] buffer.
 //  2. k_legendre_adj: b~_l = sum_rings L~_l(x_r) q_{parity(l-m)}(r) with the
-//     same monic recurrence and seeds as the synthesis; lanes evaluate rings,
-//     a 16 x 64 LDS tile per wave transposes them so lanes then own l.
+//     same monic recurrence, seeds and l-segments as the synthesis, the sum
+//     over rings on the matrix cores.
 //  3. k_adj_finish: b_lm = c_m A_l sum_groups b~ into the m-major layout.
 #include <mutex>
 
@@ -353,147 +353,207 @@ __global__ __launch_bounds__(kAdjRB) void k_ring_adjoint_cap16(LegTables t, Ring
 #define WM_ADJ_CAP_SIZES(X) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048) X(4096) X(8192)
 
 
-// b~ partial sums.  Each wave is one work item (m, ring group g) and runs
-// alone (no workgroup barrier; 4 waves per workgroup only share the launch):
-// the group's 64-ring chunks c = g, g + G, ... one after the other, for each
-// the l-range in 16-l windows.  Lanes evaluate their ring (monic
-// recurrence, 16-l chunk rescale) into the wave's 16 x 65 LDS tile, which
-// the matrix cores then multiply with the chunk's q (k_legendre_adj).  Rows
-// partial[g][off_m + l - m][k] belong to this wave only.
-constexpr int kAdjWaves = 4;  // waves per workgroup of k_legendre_adj
-
-__host__ __device__ constexpr int adj_wave_lds_doubles() {
-  return 16 * 65;  // the wave's Lambda tile
-}
-
 __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-typedef double adj_d4 __attribute__((ext_vector_type(4)));
+// x from the lane that DPP control C names.
+template <int C>
+__device__ __forceinline__ double dpp_move(double x) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, C, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), C, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (unsigned long long)lo | (unsigned long long)hi << 32);
+}
+// x of lane ^ 8 (row_ror:8) and of lane ^ 4 (row_half_mirror, then the four
+// lanes of a quad reversed).
+__device__ __forceinline__ double lane_xor8(double x) { return dpp_move<0x128>(x); }
+__device__ __forceinline__ double lane_xor4(double x) { return dpp_move<0x1b>(dpp_move<0x141>(x)); }
 
-// One pass over maps kb .. kb + KN - 1 (KN <= 4).  A 16-l window is the
-// FP64 matrix-core product D (16 l x 16 columns) = Lambda (16 l x 64 rings)
-// . Q (64 rings x 16 columns), Q's columns the real and imaginary parts of
-// the pass's maps for the even parity (columns 0 .. 2 KN - 1) and the odd
-// parity (2 KN .. 4 KN - 1); row l keeps the columns of its parity.  Sixteen
-// v_mfma_f64_16x16x4f64 per window, four rings each: lane i holds
-// A[i % 16][i / 16] = Lambda_{l0 + i % 16}(ring 4 t + i / 16) from the tile,
-// B[i / 16][i % 16] = Q[4 t + i / 16][i % 16] (the chunk's 16 B values per
-// lane stay in registers for all its windows), and D[i / 16 + 4 j][i % 16]
-// in result register j.  The sum over the chunk's 64 rings happens inside
-// the product: no cross-lane reduction.
-template <int KN>
-__global__ __launch_bounds__(64 * kAdjWaves) void k_legendre_adj(LegTables t, int G, int kb,
-                                                                 double2 *partial) {
-  static_assert(KN >= 1 && KN <= 4, "both parities of the pass's maps in 16 columns");
-  extern __shared__ double adj_lds[];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// b~ partial sums on the FP64 matrix cores.  A wave is one work item (m, ring
+// group g): units of 16 GR rings c = g, g + G, ... one after the other, for
+// each the whole l-range of the unit's rings in four segments, as in the
+// matrix-core synthesis sweep (the same segments and checkpoints).  Lane
+// 4 i + u steps segment u of ring i of every 16-ring group: with A[row][k]
+// on lane row + 4 block + 16 k that is a product, in each of the 4 blocks of
+// v_mfma_f64_4x4x4f64, of 4 l (one per segment) with 4 rings as it stands,
+// and B, 4 columns (the real and imaginary parts of 2 maps, of the step's
+// parity), has q of the same ring on lane 4 i + column: 16 distinct rings in
+// 64 lanes, so that one unit's q of both parities stays in 4 GR registers per
+// 2 maps.  The GR products of a step add up in one accumulator; the 4 blocks
+// of 4 steps are then summed by two exchange-and-add stages that leave step b
+// in block b, one row of 4 columns per lane quad.
+//
+// FP64 matrix and vector instructions share one pipe, so a step costs GR (2
+// FP64 + CG products of 16 cycles): at one map half of the 4 columns are
+// empty, where the 16 x 16 form of one row parity per column half (before)
+// left 14 of 16 empty: Nside 2048, lmax 4096, 1 map 19.0 -> 6.2 ms; Nside
+// 512, 3 maps 0.427 -> 0.28 ms.
+template <int CG, int GR>
+__global__ __launch_bounds__(64, CG == 1 ? 3 : 2) void k_legendre_adj(LegTables t, int G, int kb, int kn,
+                                                     double2 *partial) {
+  constexpr int ST = 4, RU = 16 * GR;
+  __shared__ double2 seeds[RU];  // of the unit's rings: a load where one joins would stall
+  const int lane = threadIdx.x;
   const int L = t.L, R = t.R, M = t.M, K = t.K;
-  const int64_t item = (int64_t)blockIdx.x * kAdjWaves + wv;
-  const int m = (int)(item / G), g = (int)(item - (int64_t)(item / G) * G);
-  if (m > M) return;  // the whole wave
-  double *tile = adj_lds + (size_t)wv * adj_wave_lds_doubles();  // [16][65]
+  // block b runs on XCD b % 8; runs of 8 consecutive m share an XCD, since 8
+  // entries of q (at one map) share a line
+  const int xi = blockIdx.x >> 3, g = xi % G, mi = xi / G;
+  const int m = ((mi >> 3) * 8 + (blockIdx.x & 7)) * 8 + (mi & 7);
+  if (m > M) return;
+  const int u = lane & 3, ring = lane >> 2;  // segment (and column of B), ring in a group
+  const int b = ring & 3, ds = lane >> 4;    // block, segment of the result rows
   const int64_t offm = t.off[m];
-  const int len = L - m + 1;
-  const int lp = (len + kChunk - 1) / kChunk * kChunk;
-  const double *ct = t.ctil + (offm - m);
-  const double *cs = t.cscale + offm / kChunk;
+  const double *ct0 = t.ctil + (offm - m);
+  const double *cs0 = t.cscale + offm / kChunk;
   double *prow = (double *)(partial + ((int64_t)g * t.nlpad + offm) * K + kb);
-  const int64_t rstride = 2 * (int64_t)K;  // doubles per l row of the partial sums
-  for (int j = lane; j < lp * 2 * KN; j += 64) {
-    const int l = j / (2 * KN), u = j - l * 2 * KN;
-    prow[l * rstride + u] = 0.0;
-  }
-  // this lane's B column and what it stands for
-  const int col = lane & 15, kq = lane >> 4;
-  const int cpar = col < 2 * KN ? 0 : 1;          // parity of the column
-  const int ck = (col - 2 * KN * cpar) >> 1;      // map of the column (valid if col < 4 KN)
-  const bool cval = col < 4 * KN;
-  const int nchunks = (R + 63) / 64;
-  // A wave takes its chunks g, g + G, ... two at a time: both chunks'
-  // recurrences run window by window and their products add into one
-  // accumulator, so each pass stores its rows once.  The first pass stores
-  // them outright, later passes (more than two chunks per wave) add.
+  const unsigned rstride = 2 * (unsigned)K;  // doubles per l row of the partial sums
+  const int units = (R + RU - 1) / RU;
   bool first = true;
-  for (int c0 = g; c0 < nchunks; c0 += 2 * G) {
-    double bq[2][16];
-    double x[2], prev[2] = {0.0, 0.0}, cur[2] = {0.0, 0.0};
-    int sl[2], lmin[2];
-    bool have[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int c = c0 + h * G;
-      have[h] = c < nchunks;  // wave-uniform
-      const int r = c * 64 + lane;
-      const bool ok = have[h] && r < R;
-      x[h] = ok ? t.ring_x[r] : 0.0;
-      sl[h] = ok ? t.seed_l[(int64_t)m * R + r] : kSeedNone;
-      int lm = sl[h];
-      for (int d = 32; d >= 1; d >>= 1) {
-        const int o = __shfl_xor(lm, d);
-        lm = o < lm ? o : lm;
-      }
-      lmin[h] = __builtin_amdgcn_readfirstlane(lm);
-      if (lmin[h] > L) have[h] = false;
-#pragma unroll
-      for (int tq = 0; tq < 16; ++tq) {
-        const int rg = c * 64 + 4 * tq + kq;
-        double v = 0.0;
-        if (have[h] && cval && rg < R) {
-          const double2 q = t.qbuf[q_index(rg, cpar, kb + ck, m, K, M + 1)];
-          v = (col & 1) ? q.y : q.x;
-        }
-        bq[h][tq] = v;
+  for (int c = g; c < units; c += G) {
+    const int l0 = __builtin_amdgcn_readfirstlane(
+        t.seg_l0[(int64_t)m * t.SW + c * RU / kSegRings]);
+    if (l0 > L) continue;
+    if (first) {  // rows no unit has written yet
+      for (int j = lane; j < (l0 - m) * 2 * kn; j += 64) {
+        const int l = j / (2 * kn);
+        prow[(int64_t)l * rstride + (j - l * 2 * kn)] = 0.0;
       }
     }
-    if (!have[0] && !have[1]) continue;
-    const int lstart = have[0] ? (have[1] && lmin[1] < lmin[0] ? lmin[1] : lmin[0]) : lmin[1];
-    for (int l0 = lstart; l0 <= L; l0 += kChunk) {
-      adj_d4 acc = {0.0, 0.0, 0.0, 0.0};
-      const double S = cs[(l0 - m) / kChunk];
+    const int nc = (L - l0) / kChunk + 1, ns = (nc + 3) / 4;
+    const int cb = u * ns;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (!have[h] || l0 < lmin[h]) continue;  // wave-uniform
-        // lanes = rings: L~ at l0 .. l0 + 15 into the tile (seeds sit on
-        // the 16-l grid of m)
-        const int r = (c0 + h * G) * 64 + lane;
-        if (sl[h] == l0) {
-          const double2 v = t.seed_v[(int64_t)m * R + r];
-          prev[h] = v.x;
-          cur[h] = v.y;
+    for (int i = 0; i < RU / 64; ++i) {
+      const int r = c * RU + 64 * i + lane;
+      if (r < R) seeds[64 * i + lane] = t.seed_v[(int64_t)m * R + r];
+    }
+    double x[GR], prev[GR], cur[GR], bq[2][CG][GR];
+    int sl[GR];
+#pragma unroll
+    for (int i = 0; i < GR; ++i) {
+      const int r = c * RU + 16 * i + ring;
+      const bool ok = r < R;
+      x[i] = ok ? t.ring_x[r] : 0.0;
+      sl[i] = ok ? t.seed_l[(int64_t)m * R + r] : kSeedNone;
+      double2 v = make_double2(0.0, 0.0);
+      if (ok && u > 0 && cb < nc) v = t.ckpt[((int64_t)m * 3 + u - 1) * R + r];
+      prev[i] = v.x;
+      cur[i] = v.y;
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int cg = 0; cg < CG; ++cg) {
+          const int k = 2 * cg + (u >> 1);
+          bq[p][cg][i] = ok && k < kn
+                             ? ((const double *)t.qbuf)[2 * q_index(r, p, kb + k, m, K, M + 1) + (u & 1)]
+                             : 0.0;
         }
+    }
+    const double *ct = ct0 + l0, *cs = cs0 + (l0 - m) / kChunk;
+    double *pr = prow + (int64_t)(l0 - m) * rstride + u;
+    unsigned e = kChunk * (unsigned)(cb < nc ? cb : nc - 1);
+    double cc[ST], S = cs[e / kChunk], old[CG];
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-          tile[j * 65 + lane] = cur[h];
-          const double nx = fma(x[h], cur[h], -(ct[l0 + j] * prev[h]));
-          prev[h] = cur[h];
-          cur[h] = nx;
-        }
-        prev[h] *= S;
-        cur[h] *= S;
-        wave_sync_lds();
+    for (int s = 0; s < ST; ++s) cc[s] = ct[e + s];
+    // row of the lane's results: segment ds, step b of a 4-step block; what
+    // earlier units left there is read one block ahead
+    const int drow0 = kChunk * ds * ns + b;
+    auto load_old = [&](int blk, double (&o)[CG]) {
+      const int dr = drow0 + ST * blk;
+      const bool rok = !first && ds * ns + blk / (kChunk / ST) < nc && l0 + dr <= L &&
+                       blk < ns * (kChunk / ST);
 #pragma unroll
-        for (int tq = 0; tq < 16; ++tq)
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(tile[col * 65 + 4 * tq + kq], bq[h][tq],
-                                                     acc, 0, 0, 0);
-        wave_sync_lds();  // tile reads done before the next chunk writes it
-      }
-      if (cval) {
+      for (int cg = 0; cg < CG; ++cg)
+        o[cg] = rok && 4 * cg + u < 2 * kn ? pr[(unsigned)dr * rstride + 4 * cg] : 0.0;
+    };
+    wave_sync_lds();
+    load_old(0, old);
+    for (int j = 0; j < ns; ++j) {
+      const int ls = l0 + kChunk * (cb + j);
+      bool hit = false;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int l = l0 + kq + 4 * j;
-          if (l <= L && ((l - m) & 1) == cpar) {
-            double *dst = prow + (int64_t)(l - m) * rstride + 2 * ck + (col & 1);
-            *dst = first ? acc[j] : *dst + acc[j];
+      for (int i = 0; i < GR; ++i) hit |= sl[i] == ls;
+      if (__any(hit)) {
+#pragma unroll
+        for (int i = 0; i < GR; ++i)
+          if (sl[i] == ls) {
+            const double2 v = seeds[16 * i + ring];
+            prev[i] = v.x;
+            cur[i] = v.y;
           }
-        }
       }
+      if (3 * ns + j >= nc && cb + j >= nc) {  // past the segment's rows
+#pragma unroll
+        for (int i = 0; i < GR; ++i) prev[i] = cur[i] = 0.0;
+      }
+      const unsigned en = kChunk * (unsigned)(cb + j + 1 < nc ? cb + j + 1 : nc - 1);
+      double Sn = S;
+      const int drow = drow0 + kChunk * j;
+      const bool dok = ds * ns + j < nc;
+#pragma unroll
+      for (int s0 = 0; s0 < kChunk; s0 += ST) {
+        double cn[ST], on[CG];
+#pragma unroll
+        for (int s = 0; s < ST; ++s) cn[s] = ct[(s0 + ST < kChunk ? e + s0 + ST : en) + s];
+        if (s0 + ST == kChunk) Sn = cs[en / kChunk];
+        const bool rok = dok && l0 + drow + s0 <= L;
+        const unsigned ro = (unsigned)(drow + s0) * rstride;
+        load_old(j * (kChunk / ST) + s0 / ST + 1, on);
+        __builtin_amdgcn_sched_barrier(0);
+        double d[ST][CG];
+#pragma unroll
+        for (int s = 0; s < ST; ++s)
+#pragma unroll
+          for (int cg = 0; cg < CG; ++cg) d[s][cg] = 0.0;
+        // two steps of a group at a time: their products go to two accumulators
+#pragma unroll
+        for (int s = 0; s < ST; s += 2)
+#pragma unroll
+          for (int i = 0; i < GR; ++i) {
+            const double nx = fma(x[i], cur[i], -(cc[s] * prev[i]));
+#pragma unroll
+            for (int cg = 0; cg < CG; ++cg) {
+              d[s][cg] =
+                  __builtin_amdgcn_mfma_f64_4x4x4f64(cur[i], bq[0][cg][i], d[s][cg], 0, 0, 0);
+              d[s + 1][cg] =
+                  __builtin_amdgcn_mfma_f64_4x4x4f64(nx, bq[1][cg][i], d[s + 1][cg], 0, 0, 0);
+            }
+            prev[i] = nx;
+            cur[i] = fma(x[i], nx, -(cc[s + 1] * cur[i]));
+          }
+#pragma unroll
+        for (int cg = 0; cg < CG; ++cg) {
+          const bool b2 = b & 2, b1 = b & 1;
+          const double e0 = (b2 ? d[2][cg] : d[0][cg]) + lane_xor8(b2 ? d[0][cg] : d[2][cg]);
+          const double e1 = (b2 ? d[3][cg] : d[1][cg]) + lane_xor8(b2 ? d[1][cg] : d[3][cg]);
+          const double f = (b1 ? e1 : e0) + lane_xor4(b1 ? e0 : e1);
+          if (rok && 4 * cg + u < 2 * kn) pr[ro + 4 * cg] = old[cg] + f;
+        }
+#pragma unroll
+        for (int s = 0; s < ST; ++s) cc[s] = cn[s];
+#pragma unroll
+        for (int cg = 0; cg < CG; ++cg) old[cg] = on[cg];
+      }
+#pragma unroll
+      for (int i = 0; i < GR; ++i) {
+        prev[i] *= S;
+        cur[i] *= S;
+      }
+      S = Sn;
+      e = en;
     }
+    // the next unit's segments give these rows to other lanes of the wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     first = false;
   }
+  if (first)
+    for (int j = lane; j < (L - m + 1) * 2 * kn; j += 64) {
+      const int l = j / (2 * kn);
+      prow[(int64_t)l * rstride + (j - l * 2 * kn)] = 0.0;
+    }
 }
 
 // b_lm = c_m A_l sum_g partial[g], into the m-major complex layout; one
@@ -520,13 +580,20 @@ __global__ __launch_bounds__(256) void k_adj_finish(LegTables t, int G,
   alm[idx * K + k] = acc;
 }
 
+// Rings of a work unit: 8 groups of 16 while such units fill the chip's
+// 1024 SIMDs a few times over, 4 groups below that.
+static int adjoint_unit(const LegTables &t) {
+  return (int64_t)(t.M + 1) * ((t.R + 127) / 128) >= 4096 ? 128 : 64;
+}
+
 int adjoint_groups(const LegTables &t) {
-  // one wave per (m, group): groups up to one per 64-ring chunk, while the
-  // waves stay below ~64 per CU and the partial sums below 2 GiB
-  const int nchunks = (t.R + 63) / 64;
+  // one wave per (m, group): groups up to one per unit, while the waves stay
+  // below 40 per SIMD (more only add partial sums to write and read) and the
+  // partial sums below 2 GiB
+  const int units = (t.R + adjoint_unit(t) - 1) / adjoint_unit(t);
   const double row_bytes = (double)t.nlpad * t.K * sizeof(double2);
   int G = 1;
-  while (2 * G <= nchunks && (int64_t)(t.M + 1) * 2 * G <= 16384 &&
+  while (2 * G <= units && (int64_t)(t.M + 1) * 2 * G <= 40960 &&
          row_bytes * 2 * G <= 2.0 * 1024 * 1024 * 1024)
     G *= 2;
   return G;
@@ -536,7 +603,7 @@ int adjoint_groups(const LegTables &t) {
 // (wavemoth_execute_adjoint_device_noalloc): a fixed array in device
 // memory, held by each GPU the library runs on until the process ends.
 // Every call on a GPU writes its rows before reading them (each wave of
-// k_legendre_adj zeroes its own rows first), so the contents left by an
+// k_legendre_adj writes all of its own rows), so the contents left by an
 // earlier call never matter; calls that overlap on one GPU race on it.
 constexpr size_t kAdjScratchBytes = (size_t)256 << 20;
 static __device__ __align__(256) double2 scratch[kAdjScratchBytes / sizeof(double2)];
@@ -635,21 +702,21 @@ hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  const int64_t waves = (int64_t)(t.M + 1) * G;
-  const unsigned nblk = (unsigned)((waves + kAdjWaves - 1) / kAdjWaves);
-  const size_t alds = (size_t)kAdjWaves * adj_wave_lds_doubles() * sizeof(double);
-  // passes of up to 4 maps (both parities of a pass fill the 16 columns)
-  for (int kb = 0; kb < t.K; kb += 4) {
-    const int kn = (t.K - kb) < 4 ? (t.K - kb) : 4;
-    switch (kn) {
-#define WM_ADJ_CASE(KN)                                                                   \
-  case KN:                                                                                \
-    hipLaunchKernelGGL(k_legendre_adj<KN>, dim3(nblk), dim3(64 * kAdjWaves), alds, s, t, G, kb, \
-                       partial);                                                          \
-    break;
-      WM_ADJ_CASE(1) WM_ADJ_CASE(2) WM_ADJ_CASE(3) WM_ADJ_CASE(4)
-#undef WM_ADJ_CASE
-    }
+  const unsigned nblk = (unsigned)((t.M + 64) / 64 * 64 * G);
+  // passes of up to 4 maps: 8 in one pass leave registers for half the rings
+  // only, and with them twice the partial sums to read and write (Nside 1024,
+  // 8 maps: 4.2 ms in one pass, 3.6 in two)
+  const int passes = (t.K + 3) / 4, per = (t.K + passes - 1) / passes;
+  for (int kb = 0; kb < t.K; kb += per) {
+    const int kn = std::min(per, t.K - kb);
+    const bool big = adjoint_unit(t) == 128;
+#define WM_ADJ(CG, GR)                                                                    \
+  hipLaunchKernelGGL((k_legendre_adj<CG, GR>), dim3(nblk), dim3(64), 0, s, t, G, kb, kn, partial)
+    if (kn <= 2 && big) WM_ADJ(1, 8);
+    else if (kn <= 2) WM_ADJ(1, 4);
+    else if (big) WM_ADJ(2, 8);
+    else WM_ADJ(2, 4);
+#undef WM_ADJ
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

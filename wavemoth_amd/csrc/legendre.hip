@@ -333,6 +333,11 @@ __device__ __forceinline__ void legendre_sweep(
 
 typedef double leg_d4 __attribute__((ext_vector_type(4)));
 
+// Seeds of a wave's rings in LDS (matrix-core sweep).
+__host__ __device__ constexpr int sweep_lds(int RL, int KB) {
+  return KB > kMapsVector ? 64 * RL : 1;
+}
+
 // The sweep of KB maps (even, 2 .. 16) with the contraction on the FP64
 // matrix cores.  The chunk's l-range is cut into four segments and the four
 // 16-lane rows of the wave step one segment each, all for the same rings:
@@ -359,7 +364,7 @@ __device__ __forceinline__ void legendre_sweep_mm(
     const double *__restrict__ ct, const double *__restrict__ at,
     const double *__restrict__ cs, const double *__restrict__ ring_x,
     const int *__restrict__ seed_l, const double2 *__restrict__ seed_v,
-    const double2 *__restrict__ ckpt, double2 *__restrict__ qbuf) {
+    const double2 *__restrict__ ckpt, double2 *__restrict__ qbuf, double2 *seeds) {
   constexpr int GR = 4 * RL;                      // 16-ring groups
   constexpr int C16 = KB / 8, C4 = (KB % 8) / 2;  // 16-column tiles, 4-column groups
   constexpr int B16 = C16 > 0 ? C16 : 1, B4 = C4 > 0 ? C4 : 1;
@@ -382,6 +387,12 @@ __device__ __forceinline__ void legendre_sweep_mm(
   if (l0 <= L) {
     const int nc = (L - l0) / kChunk + 1, ns = (nc + 3) / 4;  // chunks, chunks per segment
     const int cb = kq * ns;                                   // the lane's first chunk
+    // the rings' seeds wait in LDS: a load where a ring joins would stall the wave
+#pragma unroll
+    for (int i = 0; i < RL; ++i) {
+      const int r = w * 64 * RL + 64 * i + lane;
+      if (r < R) seeds[64 * i + lane] = seed_v[(int64_t)m * R + r];
+    }
 #pragma unroll
     for (int i = 0; i < GR; ++i) {
       const int r = rbase + 16 * i;
@@ -412,6 +423,9 @@ __device__ __forceinline__ void legendre_sweep_mm(
     };
     load(e, c, b16, b4);
     S = cs[e / kChunk];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     for (int j = 0; j < ns; ++j) {
       const int ls = l0 + kChunk * (cb + j);
       bool hit = false;
@@ -421,7 +435,7 @@ __device__ __forceinline__ void legendre_sweep_mm(
 #pragma unroll
         for (int i = 0; i < GR; ++i)
           if (sl[i] == ls) {
-            const double2 v = seed_v[(int64_t)m * R + rbase + 16 * i];
+            const double2 v = seeds[16 * i + col];
             prev[i] = v.x;
             cur[i] = v.y;
           }
@@ -509,7 +523,7 @@ __device__ __forceinline__ void legendre_sweep_mm(
 // and by the batched work-queue kernel.
 template <int RL, int KB>
 __device__ __forceinline__ void legendre_item(const LegTables &t, int m, int w, int kb,
-                                              int lane) {
+                                              int lane, double2 *seeds) {
   const int64_t offm = t.off[m];
   const double *at = (const double *)(t.atil + ((int64_t)kb * t.nlpad + offm - m) * KB);
   if constexpr (KB <= kMapsVector) {
@@ -524,7 +538,7 @@ __device__ __forceinline__ void legendre_item(const LegTables &t, int m, int w, 
     const int l0 = __builtin_amdgcn_readfirstlane(t.seg_l0[(int64_t)m * t.SW + sc]);
     legendre_sweep_mm<RL, KB>(t.L, t.R, t.M + 1, t.K, m, w, kb * KB, lane, l0,
                               t.ctil + (offm - m), at, t.cscale + offm / kChunk, t.ring_x,
-                              t.seed_l, t.seed_v, t.ckpt, t.qbuf);
+                              t.seed_l, t.seed_v, t.ckpt, t.qbuf, seeds);
   }
 }
 
@@ -543,7 +557,8 @@ __global__ __launch_bounds__(64) void k_legendre(LegTables t, int nkb, int bpm) 
   if (m > t.M) return;
   const int item = s % bpm;
   const int w = item / nkb, kb = item - w * nkb;
-  legendre_item<RL, KB>(t, m, w, kb, threadIdx.x);
+  __shared__ double2 seeds[sweep_lds(RL, KB)];
+  legendre_item<RL, KB>(t, m, w, kb, threadIdx.x, seeds);
 }
 
 // ------------------------------------------------------------ launchers
@@ -676,6 +691,7 @@ int batch_shape_index(int RL, int KB) {
 template <int R_, int K_>
 __global__ __launch_bounds__(256) void k_batch_legendre(BatchDev b, int first, int count,
                                                         int ctr) {
+  __shared__ double2 seeds[4][sweep_lds(R_, K_)];
   const int lane = threadIdx.x & 63;
   for (;;) {
     int it = 0;
@@ -705,7 +721,7 @@ __global__ __launch_bounds__(256) void k_batch_legendre(BatchDev b, int first, i
     t.ckpt = tp->ckpt;
     t.atil = tp->atil;
     t.qbuf = tp->qbuf;
-    legendre_item<R_, K_>(t, m, w, kb, lane);
+    legendre_item<R_, K_>(t, m, w, kb, lane, seeds[threadIdx.x >> 6]);
   }
 }
 
