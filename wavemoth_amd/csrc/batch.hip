@@ -211,7 +211,7 @@ bool ring_queues(int cus, const std::vector<const RingTables *> &rts,
     const RingTables &rt = *rts[r];
     for (int g = 0; g < rt.nlaunch; ++g) {
       if (rt.kind[g] == kRingGeneral || rt.count[g] == 0) continue;
-      const int64_t nb = ring16_blocks(rt.kind[g], rt.fftP[g], K[r], rt.count[g]);
+      const int64_t nb = ring16_blocks(rt.kind[g], rt.fftP[g], K[r], rt.count[g], sizeof(double2));
       auto &v = q16[{rt.kind[g], rt.fftP[g]}];
       for (int64_t x = 0; x < nb; ++x) v.push_back({r, g, (int)x});
     }

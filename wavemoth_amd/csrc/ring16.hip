@@ -45,7 +45,7 @@ namespace wm {
 using namespace fft;
 using fft16::pad;
 using fft16::job_slots;
-constexpr int RB = 2 * fft16::kThreads;  // threads per block of both kernels
+constexpr int RB = 2 * fft16::kThreads;  // most threads of a block
 
 __host__ __device__ inline int pow2_ceil(int v) {
   int p = 1;
@@ -110,14 +110,34 @@ __host__ __device__ constexpr bool cap_seq(int kind, int P) {
   return kind != kRingBelt16 && P / 8 > RB;
 }
 
-// Blocks of a launch: belt jobs are T = P/16 threads, cap jobs 2T threads
-// (T for cap_seq), all in 512-thread blocks.
-__host__ __device__ constexpr int ring16_jobs(int kind, int P) {
-  return kind == kRingBelt16 ? RB / (P / 16) : cap_seq(kind, P) ? 1 : RB / (P / 8);
+// Threads of a job: T = P/16 for belt jobs, 2T for cap jobs (T for cap_seq).
+__host__ __device__ constexpr int ring16_job_threads(int kind, int P) {
+  return kind == kRingBelt16 || cap_seq(kind, P) ? P / 16 : P / 8;
 }
 
-int64_t ring16_blocks(int kind, int P, int K, int count) {
-  const int J = ring16_jobs(kind, P);
+// Threads of a block, cs = size of a point.  FP64 blocks are as small as
+// their jobs allow: one wave, or one job, or one pair of belt jobs that share
+// waves (job_lane).  A CU then holds several blocks whose load, transform and
+// store phases overlap, where a single block of 512 threads idles at each of
+// its own barriers, and few rings still reach many CUs.  Measured, us of the
+// kernel with 512 threads / with this: caps P = 128 at Nside 64, 1 map 24 /
+// 16; caps P = 1024 at Nside 300, 5 maps 113 / 87; Nside 1024, 64 maps, caps
+// P = 2048 3311 / 2645, belt 3307 / 3046, wrapping rings P = 1024 1134 / 927.
+// FP32 blocks keep 512 threads: they store the maps of several jobs together.
+__host__ __device__ constexpr int ring16_threads(int kind, int P, int cs) {
+  if (cs == 8) return RB;
+  const int tj = ring16_job_threads(kind, P);
+  const int want = kind == kRingBelt16 && tj >= 64 ? 2 * tj : tj;
+  return want < 64 ? 64 : want > RB ? RB : want;
+}
+
+// Jobs of a block.
+__host__ __device__ constexpr int ring16_jobs(int kind, int P, int cs) {
+  return ring16_threads(kind, P, cs) / ring16_job_threads(kind, P);
+}
+
+int64_t ring16_blocks(int kind, int P, int K, int count, int cs) {
+  const int J = ring16_jobs(kind, P, cs);
   const int G = q_group(K), U = pow2_ceil(G);
   const int64_t ux = (int64_t)(count + 7) / 8 * q_groups(K);  // units per XCD
   if (J <= U) return 8 * ux * (U / J);
@@ -136,7 +156,7 @@ __host__ __device__ constexpr int ring16_bufs(int kind, int P, int cs) {
 }
 __host__ __device__ constexpr size_t ring16_bytes(int kind, int P, int cs) {
   return (size_t)kTwSlots * sizeof(double2) +
-         (size_t)ring16_bufs(kind, P, cs) * ring16_jobs(kind, P) * job_slots(P) * cs;
+         (size_t)ring16_bufs(kind, P, cs) * ring16_jobs(kind, P, cs) * job_slots(P) * cs;
 }
 int ring16_lds_slots(int kind, int P) {
   return (int)(ring16_bytes(kind, P, sizeof(double2)) / sizeof(double2));
@@ -401,7 +421,7 @@ __device__ __forceinline__ void belt_block_maps2(const LegTables &t, const RingT
                                                  int first, int count,
                                                  double *__restrict__ map, int b, C *lds,
                                                  const double2 *twl) {
-  constexpr int T = P / 16, J = RB / T, S = job_slots(P), h = P;
+  constexpr int T = P / 16, J = ring16_jobs(kRingBelt16, P, sizeof(C)), S = job_slots(P), h = P;
   using X = cx<C>;
   int jb, j;
   job_lane_il<T>(threadIdx.x, &jb, &j);
@@ -519,7 +539,7 @@ template <int P, typename C>
 __device__ __forceinline__ void belt_block(const LegTables &t, const RingTables &rt, int first,
                                            int count, double *__restrict__ map, int b,
                                            C *lds, const double2 *twl) {
-  constexpr int T = P / 16, J = RB / T, S = job_slots(P);
+  constexpr int T = P / 16, J = ring16_jobs(kRingBelt16, P, sizeof(C)), S = job_slots(P);
   if constexpr (sizeof(C) == 8) {
     if (t.K >= 2) {  // block-uniform
       belt_block_maps2<P>(t, rt, first, count, map, b, lds, twl);
@@ -1262,7 +1282,7 @@ template <int P, bool WRAP, typename C>
 __device__ __forceinline__ void cap_block(const LegTables &t, const RingTables &rt, int first,
                                           int count, double *__restrict__ map, int b,
                                           C *lds, const double2 *twl) {
-  constexpr int T = P / 16, J = RB / (2 * T), S = job_slots(P);
+  constexpr int T = P / 16, J = ring16_jobs(kRingCap16, P, sizeof(C)), S = job_slots(P);
   constexpr bool dual = sizeof(C) == 8;  // FP32: both rings together
   if constexpr (dual && !WRAP && J == 1) {
     if (t.K >= 2) {  // block-uniform
@@ -1340,8 +1360,10 @@ __device__ __forceinline__ void ring16_block(const LegTables &t, const RingTable
     cap_block<P, KIND == kRingWrap16>(t, rt, first, count, map, b, lds, twl);
 }
 
+template <int NB>
 __device__ __forceinline__ void load_twiddles16(double2 *twl, const double2 *__restrict__ tw) {
-  for (int u = threadIdx.x; u < kTwSlots; u += RB)
+#pragma unroll
+  for (int u = threadIdx.x; u < kTwSlots; u += NB)
     twl[u] = (u < kTwC) ? tw[u * 64] : tw[u - kTwC];
 }
 
@@ -1351,13 +1373,14 @@ __device__ __forceinline__ void load_twiddles16(double2 *twl, const double2 *__r
 template <int KIND, typename C> constexpr int ring16_waves_per_eu() { return 2; }
 
 template <int KIND, int P, typename C>
-__global__ __launch_bounds__(RB, (ring16_waves_per_eu<KIND, C>())) void k_ring16(LegTables t,
+__global__ __launch_bounds__(ring16_threads(KIND, P, sizeof(C)),
+                             (ring16_waves_per_eu<KIND, C>())) void k_ring16(LegTables t,
                                                                         RingTables rt, int first,
                                                                         int count,
                                                                         double *__restrict__ map) {
   extern __shared__ double2 lds[];
   double2 *twl = lds;
-  load_twiddles16(twl, rt.twiddle);  // first read after a barrier
+  load_twiddles16<ring16_threads(KIND, P, sizeof(C))>(twl, rt.twiddle);  // first read after a barrier
   ring16_block<KIND, P>(t, rt, first, count, map, blockIdx.x, (C *)(lds + kTwSlots), twl);
 }
 
@@ -1367,11 +1390,12 @@ __global__ __launch_bounds__(RB, (ring16_waves_per_eu<KIND, C>())) void k_ring16
 // work-queue loop: with the block body inlined into a loop the compiler kept
 // thread-invariant values live across it and spilled 12-376 bytes per lane.
 template <int KIND, int P>
-__global__ __launch_bounds__(RB, (ring16_waves_per_eu<KIND, double2>())) void k_batch_ring16(
+__global__ __launch_bounds__(ring16_threads(KIND, P, sizeof(double2)),
+                             (ring16_waves_per_eu<KIND, double2>())) void k_batch_ring16(
     BatchDev d, int first) {
   extern __shared__ double2 lds[];
   double2 *twl = lds;
-  load_twiddles16(twl, d.twiddle);
+  load_twiddles16<ring16_threads(KIND, P, sizeof(double2))>(twl, d.twiddle);
   const BatchRing16Item x = d.r16items[first + blockIdx.x];
   const LegTables &t = d.tabs[x.req];
   const RingTables &rt = d.rtabs[x.req];
@@ -1414,17 +1438,19 @@ hipError_t launch_ring16(int kind, int P, const LegTables &t, const RingTables &
   if (count <= 0) return hipSuccess;
   // FP32 belt jobs, and FP32 cap jobs of a whole block, hold two maps each at K >= 2
   const bool maps2 = (kind == kRingBelt16 ||
-                      (kind == kRingCap16 && !cap_seq(kind, P) && ring16_jobs(kind, P) == 1)) &&
+                      (kind == kRingCap16 && !cap_seq(kind, P) && ring16_jobs(kind, P, sizeof(float2)) == 1)) &&
                      t.q32 && t.K >= 2;
-  const int64_t nb = ring16_blocks(kind, P, maps2 ? (t.K + 1) / 2 : t.K, count);
-  const size_t lds = ring16_bytes(kind, P, t.q32 ? sizeof(float2) : sizeof(double2));
+  const int cs = t.q32 ? sizeof(float2) : sizeof(double2);
+  const int64_t nb = ring16_blocks(kind, P, maps2 ? (t.K + 1) / 2 : t.K, count, cs);
+  const dim3 nthr(ring16_threads(kind, P, cs));
+  const size_t lds = ring16_bytes(kind, P, cs);
 #define WM_CASE_K(KIND, PP)                                                                \
   if (kind == KIND && P == PP) {                                                           \
     if (t.q32)                                                                             \
-      hipLaunchKernelGGL((k_ring16<KIND, PP, float2>), dim3((unsigned)nb), dim3(RB), lds,  \
+      hipLaunchKernelGGL((k_ring16<KIND, PP, float2>), dim3((unsigned)nb), nthr, lds,  \
                          s, t, rt, first, count, map);                                     \
     else                                                                                   \
-      hipLaunchKernelGGL((k_ring16<KIND, PP, double2>), dim3((unsigned)nb), dim3(RB), lds, \
+      hipLaunchKernelGGL((k_ring16<KIND, PP, double2>), dim3((unsigned)nb), nthr, lds, \
                          s, t, rt, first, count, map);                                     \
     return hipGetLastError();                                                              \
   }
@@ -1441,9 +1467,10 @@ hipError_t launch_batch_ring16(int kind, int P, const BatchDev &d, int first, in
                                hipStream_t s) {
   if (count <= 0) return hipSuccess;
   const size_t lds = ring16_bytes(kind, P, sizeof(double2));
+  const dim3 nthr(ring16_threads(kind, P, sizeof(double2)));
 #define WM_CASE_K(KIND, PP)                                                                \
   if (kind == KIND && P == PP) {                                                           \
-    hipLaunchKernelGGL((k_batch_ring16<KIND, PP>), dim3((unsigned)count), dim3(RB), lds, s,  \
+    hipLaunchKernelGGL((k_batch_ring16<KIND, PP>), dim3((unsigned)count), nthr, lds, s,  \
                        d, first);                                                          \
     return hipGetLastError();                                                              \
   }

@@ -302,7 +302,7 @@ hipError_t ring_set_lds_limit(int slots);
 // Register-FFT ring kernels (ring16.hip) for FFT lengths P = 16 .. 4096.
 bool ring16_size_ok(int P);
 int ring16_lds_slots(int kind, int P);
-int64_t ring16_blocks(int kind, int P, int K, int count);
+int64_t ring16_blocks(int kind, int P, int K, int count, int cs);
 hipError_t ring16_set_lds_limits();
 hipError_t launch_ring16(int kind, int P, const LegTables &t, const RingTables &rt, int first,
                          int count, double *map, hipStream_t s);
