@@ -29,24 +29,27 @@ namespace wm {
 
 using namespace fft;
 
-// MAXP: the plan's longest transform (Bluestein length, or twice a power-of-
-// two ring's h); the per-thread loops and FFT passes are sized for it.
+// One block per (ring pair, map), the maps of a q group on one XCD.  MAXP: the
+// plan's longest transform (Bluestein length, or twice a power-of-two ring's
+// h); the per-thread loops and FFT passes are sized for it.
 template <int MAXP>
 __global__ __launch_bounds__(NT) void k_ring_adjoint(LegTables t, RingTables rt, int first,
-                                                     int lds_slots,
+                                                     int count, int lds_slots,
                                                      const double *__restrict__ map) {
   constexpr int kHalf = (MAXP / 2 + 1 + NT - 1) / NT;  // h-range entries per thread
   constexpr int kFull = (MAXP + NT - 1) / NT;          // P-range entries per thread
   extern __shared__ double2 lds[];
   double2 *twl = lds + lds_slots - kTwSlots;
-  const RingPair rp = rt.pairs[rt.order[first + blockIdx.x]];
+  int pi, k;
+  if (!ring16_job(blockIdx.x, 1, 0, t.K, count, &pi, &k)) return;
+  const RingPair rp = rt.pairs[rt.order[first + pi]];
   const int n = rp.n, h = n / 2, K = t.K, M = t.M, P = rp.P;
   const bool south = rp.pix_s >= 0;
   const double2 *chirp = rt.chirp + rp.chirp_off;
   const double2 *vhat = rt.vhat + rp.vhat_off;
   load_twiddles(twl, rt.twiddle);
   const int nhemi = south ? 2 : 1;
-  for (int k = 0; k < K; ++k) {
+  {
     double2 *qe = t.qbuf + q_index(rp.r, 0, k, 0, K, M + 1);  // element m at [m * G]
     double2 *qo = t.qbuf + q_index(rp.r, 1, k, 0, K, M + 1);
     for (int hemi = 0; hemi < nhemi; ++hemi) {
@@ -149,7 +152,7 @@ __global__ __launch_bounds__(NT) void k_ring_adjoint(LegTables t, RingTables rt,
 
 // The ring adjoint of power-of-two rings with mmax <= h (the forward belt
 // kernel's rings) on the register FFT: a job of T = h/16 threads per (ring
-// pair, map), 512-thread blocks.  Per hemisphere: z_p = g_{2p} + i g_{2p+1}
+// pair, map).  Per hemisphere: z_p = g_{2p} + i g_{2p+1}
 // for p = j + T rho, Z = DFT_h(z) in registers (canonical layout), Z into the
 // job's buffer and back for the partner Z_{h-k}, then for the thread's own
 // k = j + T rho
@@ -157,11 +160,19 @@ __global__ __launch_bounds__(NT) void k_ring_adjoint(LegTables t, RingTables rt,
 // (Z_h = Z_0; thread 0 also forms G^_h), F_m = e^{-i pi s m/n} G^_m for
 // m = k <= mmax, and q_e = F_N + F_S, q_o = F_N - F_S (the southern pass
 // adds to what the same thread wrote for the northern ring).
-constexpr int kAdjRB = 2 * fft16::kThreads;  // threads per block
-
-__host__ __device__ constexpr size_t adj16_bytes(int P) {
-  return (size_t)kTwSlots * sizeof(double2) +
-         (size_t)(kAdjRB / (P / 16)) * fft16::job_slots(P) * sizeof(double2);
+// Blocks hold at least one wave and `maps` jobs where they fit in 512 threads,
+// so that a few rings still reach many CUs and several blocks share one.  The
+// belt takes all maps of a q group (they share lines of q and of the map:
+// 3 maps at Nside 512 64 us, 79 with one job per block), the caps, whose time
+// is in their transforms, one job (52 us, 60 with the group's).
+constexpr int kAdjRB = 2 * fft16::kThreads;  // most threads per block
+inline int adj16_threads(int P, int maps) {
+  int n = P / 16;
+  while (n < kAdjRB && (n < 64 || n / (P / 16) < maps)) n *= 2;
+  return n;
+}
+constexpr size_t adj16_bytes(int P, int threads) {
+  return (size_t)(kTwSlots + threads / (P / 16) * fft16::job_slots(P)) * sizeof(double2);
 }
 
 template <int P>
@@ -169,19 +180,22 @@ __global__ __launch_bounds__(kAdjRB) void k_ring_adjoint16(LegTables t, RingTabl
                                                            int count,
                                                            const double *__restrict__ map) {
   using fft16::pad;
-  constexpr int T = P / 16, J = kAdjRB / T;
+  constexpr int T = P / 16;
+  const int J = blockDim.x / T;
   extern __shared__ double2 lds[];
   double2 *twl = lds;
-  for (int u = threadIdx.x; u < kTwSlots; u += kAdjRB)  // read after the FFT's first barrier
+  for (int u = threadIdx.x; u < kTwSlots; u += blockDim.x)  // read after the FFT's first barrier
     twl[u] = (u < kTwC) ? rt.twiddle[u * 64] : rt.twiddle[u - kTwC];
   const int jb = threadIdx.x / T;
   int j = threadIdx.x - jb * T;
   double2 *buf = lds + kTwSlots + jb * fft16::job_slots(P);
   const int K = t.K, M = t.M;
-  const int64_t g = (int64_t)blockIdx.x * J + jb;
-  const int pi = (int)(g / K), k = (int)(g - (int64_t)(g / K) * K);
-  const bool act = pi < count;
-  const RingPair rp = rt.pairs[rt.order[first + (act ? pi : 0)]];
+  int pi, k;
+  // a job is padding only if every later one of its block is
+  if (!ring16_job(blockIdx.x, J, 0, K, count, &pi, &k)) return;
+  const bool act = ring16_job(blockIdx.x, J, jb, K, count, &pi, &k);
+  if (!act) pi = k = 0;
+  const RingPair rp = rt.pairs[rt.order[first + pi]];
   const int n = rp.n;
   const bool south = rp.pix_s >= 0;
   double2 *qe = t.qbuf + q_index(rp.r, 0, k, 0, K, M + 1);
@@ -258,19 +272,22 @@ __global__ __launch_bounds__(kAdjRB) void k_ring_adjoint_cap16(LegTables t, Ring
                                                                int first, int count,
                                                                const double *__restrict__ map) {
   using fft16::pad;
-  constexpr int T = P / 16, J = kAdjRB / T;
+  constexpr int T = P / 16;
+  const int J = blockDim.x / T;
   extern __shared__ double2 lds[];
   double2 *twl = lds;
-  for (int u = threadIdx.x; u < kTwSlots; u += kAdjRB)  // read after the FFT's first barrier
+  for (int u = threadIdx.x; u < kTwSlots; u += blockDim.x)  // read after the FFT's first barrier
     twl[u] = (u < kTwC) ? rt.twiddle[u * 64] : rt.twiddle[u - kTwC];
   const int jb = threadIdx.x / T;
   int j = threadIdx.x - jb * T;
   double2 *buf = lds + kTwSlots + jb * fft16::job_slots(P);
   const int K = t.K, M = t.M;
-  const int64_t g = (int64_t)blockIdx.x * J + jb;
-  const int pi = (int)(g / K), k = (int)(g - (int64_t)(g / K) * K);
-  const bool act = pi < count;
-  const RingPair rp = rt.pairs[rt.order[first + (act ? pi : 0)]];
+  int pi, k;
+  // a job is padding only if every later one of its block is
+  if (!ring16_job(blockIdx.x, J, 0, K, count, &pi, &k)) return;
+  const bool act = ring16_job(blockIdx.x, J, jb, K, count, &pi, &k);
+  if (!act) pi = k = 0;
+  const RingPair rp = rt.pairs[rt.order[first + pi]];
   const int n = rp.n, h = n / 2;
   const bool south = rp.pix_s >= 0;
   const double2 *chirp = rt.chirp + rp.chirp_off;  // [h]
@@ -650,12 +667,12 @@ hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double
     if (rt.count[i] == 0) continue;
     if (rt.kind[i] == kRingBelt16 && rt.fftP[i] <= 4096) {
       // power-of-two rings with mmax <= h: the register-FFT adjoint
-      const int P = rt.fftP[i], J = kAdjRB / (P / 16);
-      const unsigned nb = (unsigned)(((int64_t)rt.count[i] * t.K + J - 1) / J);
+      const int P = rt.fftP[i], nthr = adj16_threads(P, pow2_ceil(q_group(t.K)));
+      const unsigned nb = (unsigned)ring16_job_blocks(nthr / (P / 16), t.K, rt.count[i]);
       switch (P) {
 #define WM_ADJ16_CASE(PP)                                                                   \
   case PP:                                                                                  \
-    hipLaunchKernelGGL(k_ring_adjoint16<PP>, dim3(nb), dim3(kAdjRB), adj16_bytes(PP), s, t,  \
+    hipLaunchKernelGGL(k_ring_adjoint16<PP>, dim3(nb), dim3(nthr), adj16_bytes(PP, nthr), s, t,  \
                        rt, rt.first[i], rt.count[i], map);                                  \
     break;
         WM_ADJ16_SIZES(WM_ADJ16_CASE)
@@ -669,12 +686,12 @@ hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double
     }
     if (rt.kind[i] == kRingCap16 && 2 * rt.fftP[i] >= 32 && 2 * rt.fftP[i] <= 8192) {
       // the cap kernel's rings: Bluestein of length P = 2 P2 on the register FFT
-      const int P = 2 * rt.fftP[i], J = kAdjRB / (P / 16);
-      const unsigned nb = (unsigned)(((int64_t)rt.count[i] * t.K + J - 1) / J);
+      const int P = 2 * rt.fftP[i], nthr = adj16_threads(P, 1);
+      const unsigned nb = (unsigned)ring16_job_blocks(nthr / (P / 16), t.K, rt.count[i]);
       switch (P) {
 #define WM_ADJCAP_CASE(PP)                                                                  \
   case PP:                                                                                  \
-    hipLaunchKernelGGL(k_ring_adjoint_cap16<PP>, dim3(nb), dim3(kAdjRB), adj16_bytes(PP), s, \
+    hipLaunchKernelGGL(k_ring_adjoint_cap16<PP>, dim3(nb), dim3(nthr), adj16_bytes(PP, nthr), s, \
                        t, rt, rt.first[i], rt.count[i], map);                               \
     break;
         WM_ADJ_CAP_SIZES(WM_ADJCAP_CASE)
@@ -691,8 +708,9 @@ hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double
     switch (rt.adj_maxp) {
 #define WM_RADJ(MP)                                                                         \
   case MP:                                                                                  \
-    hipLaunchKernelGGL(k_ring_adjoint<MP>, dim3(rt.count[i]), dim3(NT), lds, s, t, rt,      \
-                       rt.first[i], rt.adj_lds[i], map);                                    \
+    hipLaunchKernelGGL(k_ring_adjoint<MP>,                                                  \
+                       dim3((unsigned)ring16_job_blocks(1, t.K, rt.count[i])), dim3(NT),    \
+                       lds, s, t, rt, rt.first[i], rt.count[i], rt.adj_lds[i], map);        \
     break;
       WM_RADJ(1024) WM_RADJ(2048) WM_RADJ(4096) WM_RADJ(8192)
 #undef WM_RADJ
@@ -741,13 +759,15 @@ hipError_t adjoint_set_lds_limit(int slots) {
 #define WM_ADJ16_SET(PP)                                                                    \
   if (e == hipSuccess)                                                                      \
     e = hipFuncSetAttribute((const void *)k_ring_adjoint16<PP>,                             \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)adj16_bytes(PP));
+                            hipFuncAttributeMaxDynamicSharedMemorySize,             \
+                            (int)adj16_bytes(PP, kAdjRB));
   WM_ADJ16_SIZES(WM_ADJ16_SET)
 #undef WM_ADJ16_SET
 #define WM_ADJCAP_SET(PP)                                                                   \
   if (e == hipSuccess)                                                                      \
     e = hipFuncSetAttribute((const void *)k_ring_adjoint_cap16<PP>,                         \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)adj16_bytes(PP));
+                            hipFuncAttributeMaxDynamicSharedMemorySize,             \
+                            (int)adj16_bytes(PP, kAdjRB));
   WM_ADJ_CAP_SIZES(WM_ADJCAP_SET)
 #undef WM_ADJCAP_SET
   if (e == hipSuccess) cur = slots;

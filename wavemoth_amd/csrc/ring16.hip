@@ -47,37 +47,6 @@ using fft16::pad;
 using fft16::job_slots;
 constexpr int RB = 2 * fft16::kThreads;  // most threads of a block
 
-__host__ __device__ inline int pow2_ceil(int v) {
-  int p = 1;
-  while (p < v) p <<= 1;
-  return p;
-}
-
-// Job (pair index, map) of job slot jb of block b.  U = pow2_ceil(q_group(K))
-// jobs per unit (pair, q group), J jobs per block.  Block b runs on XCD
-// x = b mod 8; the units of XCD x are pairs x, x + 8, ..., each with all its
-// q groups, so that every line of a pair's pixel rows (all maps of a pixel)
-// is written through one L2.  Returns false for a padding job.
-__device__ __forceinline__ bool ring16_job(int b, int J, int jb, int K, int count, int *pi,
-                                           int *k) {
-  const int G = q_group(K), nG = q_groups(K), U = pow2_ceil(G);
-  const int x = b & 7, s = b >> 3;
-  int sg, u;  // unit index on XCD x, job in unit
-  if (J <= U) {
-    const int BU = U / J;  // blocks per unit, consecutive on XCD x
-    sg = s / BU;
-    u = (s - sg * BU) * J + jb;
-  } else {
-    const int UB = J / U;  // units per block
-    sg = s * UB + jb / U;
-    u = jb & (U - 1);
-  }
-  const int q = sg / nG;
-  *pi = q * 8 + x;
-  *k = (sg - q * nG) * G + u;
-  return *pi < count && u < G && *k < K;
-}
-
 // Entry e (< 8) of the complex values a thread of a cap_seq job parks in
 // its own map column `col` (stride K doubles) of a ring's pixel rows: an FP64
 // value in rows (2 e) T + tt and (2 e + 1) T + tt, an FP32 one in row
@@ -137,14 +106,8 @@ __host__ __device__ constexpr int ring16_jobs(int kind, int P, int cs) {
 }
 
 int64_t ring16_blocks(int kind, int P, int K, int count, int cs) {
-  const int J = ring16_jobs(kind, P, cs);
-  const int G = q_group(K), U = pow2_ceil(G);
-  const int64_t ux = (int64_t)(count + 7) / 8 * q_groups(K);  // units per XCD
-  if (J <= U) return 8 * ux * (U / J);
-  const int UB = J / U;
-  return 8 * ((ux + UB - 1) / UB);
+  return ring16_job_blocks(ring16_jobs(kind, P, cs), K, count);
 }
-
 
 // LDS of one block: the twiddle table (double2) first, then the jobs'
 // buffers of cs-byte points
@@ -1352,6 +1315,12 @@ template <int KIND, int P, typename C>
 __device__ __forceinline__ void ring16_block(const LegTables &t, const RingTables &rt, int first,
                                              int count, double *__restrict__ map, int b,
                                              C *lds, const double2 *twl) {
+  if constexpr (sizeof(C) == 16) {
+    // a block of padding jobs only (K maps fill up to a power of two of
+    // jobs): a job is padding only if every later one of its block is
+    int pi, k;
+    if (!ring16_job(b, ring16_jobs(KIND, P, sizeof(C)), 0, t.K, count, &pi, &k)) return;
+  }
   if constexpr (KIND == kRingBelt16)
     belt_block<P>(t, rt, first, count, map, b, lds, twl);
   else if constexpr (cap_seq(KIND, P))

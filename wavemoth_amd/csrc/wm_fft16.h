@@ -174,4 +174,45 @@ __device__ __forceinline__ void fft2(C (&v)[2][16], C *buf0, C *buf1, const doub
 }
 
 }  // namespace fft16
+
+__host__ __device__ inline int pow2_ceil(int v) {
+  int p = 1;
+  while (p < v) p <<= 1;
+  return p;
+}
+
+// Job (pair index, map) of job slot jb of block b.  U = pow2_ceil(q_group(K))
+// jobs per unit (pair, q group), J jobs per block.  Block b runs on XCD
+// x = b mod 8; the units of XCD x are pairs x, x + 8, ..., each with all its
+// q groups, so that every line of a pair's pixel rows (all maps of a pixel)
+// is written through one L2.  Returns false for a padding job.
+__device__ __forceinline__ bool ring16_job(int b, int J, int jb, int K, int count, int *pi,
+                                           int *k) {
+  const int G = q_group(K), nG = q_groups(K), U = pow2_ceil(G);
+  const int x = b & 7, s = b >> 3;
+  int sg, u;  // unit index on XCD x, job in unit
+  if (J <= U) {
+    const int BU = U / J;  // blocks per unit, consecutive on XCD x
+    sg = s / BU;
+    u = (s - sg * BU) * J + jb;
+  } else {
+    const int UB = J / U;  // units per block
+    sg = s * UB + jb / U;
+    u = jb & (U - 1);
+  }
+  const int q = sg / nG;
+  *pi = q * 8 + x;
+  *k = (sg - q * nG) * G + u;
+  return *pi < count && u < G && *k < K;
+}
+
+// Blocks of a launch over `count` pairs of K maps with J jobs per block.
+inline int64_t ring16_job_blocks(int J, int K, int count) {
+  const int U = pow2_ceil(q_group(K));
+  const int64_t ux = (int64_t)(count + 7) / 8 * q_groups(K);  // units per XCD
+  if (J <= U) return 8 * ux * (U / J);
+  const int UB = J / U;
+  return 8 * ((ux + UB - 1) / UB);
+}
+
 }  // namespace wm
