@@ -150,7 +150,7 @@ __global__ __launch_bounds__(NT) void k_ring_adjoint(LegTables t, RingTables rt,
   }
 }
 
-// The ring adjoint of power-of-two rings with mmax <= h (the forward belt
+// The ring adjoint of power-of-two rings with mmax < n (the forward belt
 // kernel's rings) on the register FFT: a job of T = h/16 threads per (ring
 // pair, map).  Per hemisphere: z_p = g_{2p} + i g_{2p+1}
 // for p = j + T rho, Z = DFT_h(z) in registers (canonical layout), Z into the
@@ -201,6 +201,16 @@ __global__ __launch_bounds__(kAdjRB) void k_ring_adjoint16(LegTables t, RingTabl
   double2 *qe = t.qbuf + q_index(rp.r, 0, k, 0, K, M + 1);
   double2 *qo = t.qbuf + q_index(rp.r, 1, k, 0, K, M + 1);
   const int64_t qs = q_group(K);
+  auto put = [&](int m, double2 f, int hemi) {
+    const int64_t o = (int64_t)m * qs;
+    if (hemi == 0) {
+      qe[o] = f;
+      qo[o] = f;
+    } else {
+      qe[o] = cadd(qe[o], f);
+      qo[o] = csub(qo[o], f);
+    }
+  };
 #pragma unroll 1
   for (int hemi = 0; hemi < 2; ++hemi) {  // every job takes both passes (block barriers)
     const bool on = act && (hemi == 0 || south);
@@ -226,16 +236,11 @@ __global__ __launch_bounds__(kAdjRB) void k_ring_adjoint16(LegTables t, RingTabl
       const double2 e = cadd(za, cconj(zc)), d = csub(za, cconj(zc));
       const double2 od = cmul(om, d);
       const double2 gk = make_double2(0.5 * (e.x + od.y), 0.5 * (e.y - od.x));
-      if (on && kk <= M) {
-        const double2 f = cmul(gk, w);
-        const int64_t o = (int64_t)kk * qs;
-        if (hemi == 0) {
-          qe[o] = f;
-          qo[o] = f;
-        } else {
-          qe[o] = cadd(qe[o], f);
-          qo[o] = csub(qo[o], f);
-        }
+      if (on && kk <= M) put(kk, cmul(gk, w), hemi);
+      // m = n - k past h: G^_m = conj G^_k, e^{-i pi s m/n} = (-1)^s conj w
+      if (on && kk > 0 && n - kk <= M) {
+        const double2 f = cconj(cmul(gk, w));
+        put(n - kk, rp.s ? make_double2(-f.x, -f.y) : f, hemi);
       }
       w = cmul(w, wstep);
       om = cmul(om, ostep);
@@ -245,15 +250,7 @@ __global__ __launch_bounds__(kAdjRB) void k_ring_adjoint16(LegTables t, RingTabl
       const double2 z0 = v[0];
       const double2 e = cadd(z0, cconj(z0)), d = csub(z0, cconj(z0));
       const double2 gh = make_double2(0.5 * (e.x - d.y), 0.5 * (e.y + d.x));
-      const double2 f = cmul(gh, expipi(-(int64_t)rp.s * P, n));
-      const int64_t o = (int64_t)P * qs;
-      if (hemi == 0) {
-        qe[o] = f;
-        qo[o] = f;
-      } else {
-        qe[o] = cadd(qe[o], f);
-        qo[o] = csub(qo[o], f);
-      }
+      put(P, cmul(gh, expipi(-(int64_t)rp.s * P, n)), hemi);
     }
   }
 }
@@ -666,7 +663,7 @@ hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double
   for (int i = 0; i < rt.nlaunch; ++i) {
     if (rt.count[i] == 0) continue;
     if (rt.kind[i] == kRingBelt16 && rt.fftP[i] <= 4096) {
-      // power-of-two rings with mmax <= h: the register-FFT adjoint
+      // the forward belt kernel's rings: the register-FFT adjoint
       const int P = rt.fftP[i], nthr = adj16_threads(P, pow2_ceil(q_group(t.K)));
       const unsigned nb = (unsigned)ring16_job_blocks(nthr / (P / 16), t.K, rt.count[i]);
       switch (P) {

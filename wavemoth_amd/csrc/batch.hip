@@ -163,7 +163,7 @@ Geometry *get_geometry(wavemoth_batch b, int N, int L, int M) {
 bool ensure_rings(wavemoth_batch b, Geometry *g, int w) {
   if (g->have_rt[w]) return true;
   if (!build_ring_geometry(b->arena, g->rt[w], g->rhost[w], g->N, g->M, true, w == 1,
-                           b->stream))
+                           true, b->stream))
     return false;
   if (!g->rhost[w].lr.groups.empty()) {  // none up to Nside kMaxNside
     set_err("batch: rings longer than the register-FFT kernels hold");

@@ -379,7 +379,7 @@ namespace wm {
 static bool general_fits(int h, int P) { return P == 0 ? h <= kMaxFFT / 2 : P <= kMaxFFT; }
 
 bool build_ring_geometry(DevArena &a, RingTables &rt, RingHost &host, int N, int M,
-                         bool phase_shifts, bool wide, hipStream_t stream) {
+                         bool phase_shifts, bool wide, bool fp64, hipStream_t stream) {
   const int nrings = 4 * N - 1, mid = 2 * N - 1, R = 2 * N;
   // Ring length of iring and phi0 = pi * num / den of grid entry iring
   // (src/wavemoth.c:1199-1232); den always equals the ring length.
@@ -435,8 +435,12 @@ bool build_ring_geometry(DevArena &a, RingTables &rt, RingHost &host, int N, int
       rp.P = next_pow2(2 * h - 1);
       cost[r] = 2.0 * (double)rp.P * std::log2((double)rp.P) + (double)(M + 1);
     }
-    if (is_pow2(h) && M <= h && ring16_size_ok(h)) {
-      // non-aliasing power-of-two ring: one FFT of h points
+    if (is_pow2(h) && (M <= h || (fp64 && M < n && h <= 4096)) && ring16_size_ok(h)) {
+      // power-of-two ring, one FFT of h points: no wrap, or in FP64 one
+      // conjugate term per bin (mmax < n).  Ring stage at lmax = 3 Nside - 1,
+      // these rings in the general kernel or the split Bluestein / here:
+      // Nside 1024, 3 maps 807 / 575 us, 16 maps 3.16 / 2.29 ms; Nside 2048,
+      // 1 map 982 / 789 us
       kind[r] = kRingBelt16;
       fftP[r] = h;
     } else if (n % 4 == 0) {
@@ -682,7 +686,7 @@ bool build_ring_geometry(DevArena &a, RingTables &rt, RingHost &host, int N, int
 
 static bool build_ring_tables(wavemoth_plan p) {
   if (!build_ring_geometry(p->arena, p->rt, p->rhost, p->N, p->M, p->phase_shifts,
-                           p->K >= kRingWideMaps, p->stream))
+                           p->K >= kRingWideMaps, p->mix < 0, p->stream))
     return false;
   p->npix = p->rhost.npix;
   return true;

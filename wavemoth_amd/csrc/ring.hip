@@ -23,6 +23,7 @@
 // conjugate tabulated per h at plan time.  LDS arrays are padded by one
 // slot per 8 (pidx) so the Stockham writes of the first passes do not pile
 // onto one bank.
+#include <algorithm>
 #include <mutex>
 
 #include "wm_fft.h"
@@ -51,10 +52,12 @@ __device__ __forceinline__ void store_pix2(double *out, int p, double2 z, int os
 // MAXP: the size class (>= the ring's Bluestein P and n = 2h, see
 // ring_class); the per-thread bin, pair, output and staging counts follow
 // from it, the twiddle table stays the kMaxFFT one.
+// hemi0 .. hemi1: the hemispheres to transform (0 north, 1 south), as far as
+// the pair has them.
 template <typename Q, int MAXP = kMaxFFT>
 __device__ __forceinline__ void ring_pair_body(const LegTables &t, const RingTables &rt, int pair, int k,
                                double2 *lds, int lds_slots, double *__restrict__ outk,
-                               int ostride) {
+                               int ostride, int hemi0 = 0, int hemi1 = 1) {
   constexpr int kBins = (MAXP / 2 + 1 + NT - 1) / NT;   // bins 0 .. h per thread
   constexpr int kPairs = (MAXP / 4 + 1 + NT - 1) / NT;  // Z pairs per thread
   constexpr int kOut = (MAXP / 2 + NT - 1) / NT;        // output pairs per thread
@@ -77,9 +80,9 @@ __device__ __forceinline__ void ring_pair_body(const LegTables &t, const RingTab
   const int J = (M + h) / n + 2;   // j runs over [0, J)
   const int JG = (J + G - 1) / G;  // j-iterations per group
 
-  const int nhemi = south ? 2 : 1;
+  if (!south) hemi1 = 0;
   {
-    for (int hemi = 0; hemi < nhemi; ++hemi) {
+    for (int hemi = hemi0; hemi <= hemi1; ++hemi) {
       // Opaque copy of the thread index: keeps the per-bin LDS/global
       // addresses from being hoisted out of the map/hemisphere loops (they
       // would stay live across the FFTs and spill).
@@ -224,24 +227,26 @@ __device__ __forceinline__ void ring_pair_body(const LegTables &t, const RingTab
   }
 }
 
-// Block -> (ring pair, map).  The G = q_group(K) maps of one q group share
-// its 128-byte lines, so their G workgroups are put on one XCD (hardware
-// dispatches block b to XCD b % 8) at consecutive dispatch slots: block
-// b = 8 (sigma G + j) + x runs map j of group gamma = 8 sigma + x, where
-// gamma enumerates (ring pair i, map group).
+// Block -> (ring pair, map), and with split the hemisphere.  The G =
+// q_group(K) maps of one q group share its 128-byte lines, so their (split: 2)
+// G workgroups are put on one XCD (hardware dispatches block b to XCD b % 8)
+// at consecutive dispatch slots: block b = 8 (sigma G + j) + x runs map j of
+// group gamma = 8 sigma + x, where gamma enumerates (ring pair i, map group).
 template <typename Q, int MAXP>
 __global__ __launch_bounds__(NT) void k_ring_pairs(LegTables t, RingTables rt, int first,
-                                                   int count, int lds_slots,
+                                                   int count, int lds_slots, int split,
                                                    double *__restrict__ map) {
   extern __shared__ double2 lds[];
   const int K = t.K, G = q_group(K), nG = q_groups(K);
-  const int b = blockIdx.x, x = b & 7, s = b >> 3;
+  const int b = blockIdx.x, x = b & 7, s = (b >> 3) >> split;
+  const int hemi = split & (b >> 3);
   const int sigma = s / G, j = s - sigma * G;
   const int gamma = sigma * 8 + x;
   const int i = gamma / nG, k = (gamma - i * nG) * G + j;
   if (i >= count || k >= K) return;
   load_twiddles(lds + lds_slots - kTwSlots, rt.twiddle);
-  ring_pair_body<Q, MAXP>(t, rt, rt.order[first + i], k, lds, lds_slots, map + k, K);
+  ring_pair_body<Q, MAXP>(t, rt, rt.order[first + i], k, lds, lds_slots, map + k, K, hemi,
+                          split ? hemi : 1);
 }
 
 // Ring stage of a batch in the general kernel: block i runs item
@@ -378,6 +383,7 @@ hipError_t launch_ring_synth(const LegTables &t, const RingTables &rt, double *m
   for (int i = 0; i < rt.nlaunch; ++i) {
     // the long path (launch_long_rings) runs the kRingLong groups
     if (rt.count[i] == 0 || rt.kind[i] == kRingLong) continue;
+    if (!t.q32 && ring16_small(rt.kind[i], rt.fftP[i])) continue;  // below
     hipError_t e;
     if (rt.kind[i] != kRingGeneral) {
       e = launch_ring16(rt.kind[i], rt.fftP[i], t, rt, rt.first[i], rt.count[i], map, s);
@@ -385,16 +391,23 @@ hipError_t launch_ring_synth(const LegTables &t, const RingTables &rt, double *m
       // a general group's fftP is its size class (ring_class of its pairs)
       const size_t lds = (size_t)rt.lds[i] * sizeof(double2);
       const int64_t groups = (int64_t)rt.count[i] * q_groups(t.K);
-      const int64_t nb = (groups + 7) / 8 * 8 * q_group(t.K);
+      // A workgroup per hemisphere where a workgroup per pair leaves some of
+      // the chip's 256 CUs with room (both read the pair's q; otherwise the
+      // hemispheres run one after the other).  Measured, us, together / split:
+      // 32 workgroups 15.4 / 9.6, 256 48 / 32, 640 34 / 31; at one full round
+      // (512 of 72 KB) 125 / 132.
+      const int64_t room = 256 * std::min<int64_t>(4, 160 * 1024 / std::max<size_t>(lds, 1));
+      const int split = groups * q_group(t.K) < room ? 1 : 0;
+      const int64_t nb = ((groups + 7) / 8 * 8 * q_group(t.K)) << split;
       switch (rt.fftP[i]) {
 #define WM_RP(MP)                                                                           \
   case MP:                                                                                  \
     if (t.q32)                                                                              \
       hipLaunchKernelGGL((k_ring_pairs<float2, MP>), dim3((unsigned)nb), dim3(NT), lds, s, t, \
-                         rt, rt.first[i], rt.count[i], rt.lds[i], map);                     \
+                         rt, rt.first[i], rt.count[i], rt.lds[i], split, map);              \
     else                                                                                    \
       hipLaunchKernelGGL((k_ring_pairs<double2, MP>), dim3((unsigned)nb), dim3(NT), lds, s,   \
-                         t, rt, rt.first[i], rt.count[i], rt.lds[i], map);                  \
+                         t, rt, rt.first[i], rt.count[i], rt.lds[i], split, map);           \
     break;
         WM_RP(1024) WM_RP(2048) WM_RP(4096) WM_RP(8192)
 #undef WM_RP
@@ -405,7 +418,7 @@ hipError_t launch_ring_synth(const LegTables &t, const RingTables &rt, double *m
     }
     if (e != hipSuccess) return e;
   }
-  return hipSuccess;
+  return t.q32 ? hipSuccess : launch_ring16_small(t, rt, map, s);
 }
 
 }  // namespace wm

@@ -4,9 +4,9 @@
 // length n (imaginary parts of DC and Nyquist ignored, unnormalised), with
 // the same Z-pair reduction of the c2r to a complex DFT of h = n/2.
 //
-// kind 1, belt: h a power of two and mmax <= h (the equatorial belt): one
-//   job per (ring pair, map), both rings from one read of E and O, one
-//   P = h point inverse FFT per ring.
+// kind 1, belt: h a power of two and mmax <= h (the equatorial belt; in FP64
+//   mmax < n for h <= 4096): one job per (ring pair, map), both rings from one
+//   read of E and O, one P = h point inverse FFT per ring.
 // kind 2, caps: h = 2i not a power of two, 4i > mmax (no wrap: bin b
 //   receives at most g_b and the conjugate term (-1)^s conj g_{n-b}, so the
 //   fold is two passes over LDS with one writer per bin): the length-h
@@ -103,6 +103,22 @@ __host__ __device__ constexpr int ring16_threads(int kind, int P, int cs) {
 // Jobs of a block.
 __host__ __device__ constexpr int ring16_jobs(int kind, int P, int cs) {
   return ring16_threads(kind, P, cs) / ring16_job_threads(kind, P);
+}
+
+// Threads that share a block's jobs and meet at its barriers.
+template <int P, typename C>
+__host__ __device__ constexpr int belt_nt() {
+  return ring16_threads(kRingBelt16, P, sizeof(C));
+}
+template <int P, typename C>
+__host__ __device__ constexpr int cap_nt() {
+  return ring16_threads(kRingCap16, P, sizeof(C));
+}
+// This thread's index among them (k_ring16_small runs one-wave blocks side
+// by side in one workgroup).
+template <int NT>
+__device__ __forceinline__ int job_tid() {
+  return NT <= 64 ? threadIdx.x & 63 : threadIdx.x;
 }
 
 int64_t ring16_blocks(int kind, int P, int K, int count, int cs) {
@@ -206,7 +222,7 @@ __device__ __forceinline__ void belt_fft_out(C *buf, const double2 *twl, int j, 
       om = cmul(om, ostep);
     }
   }
-  fft16::fft<P, true>(v, buf, twl, j);
+  fft16::fft<P, true, belt_nt<P, C>()>(v, buf, twl, j);
   if (on) put16<T>(out, j, v, K);
 }
 
@@ -237,6 +253,28 @@ __device__ __forceinline__ void belt_pair(const RingPair &rp, const C *__restric
     for (int rho = 0; rho < 16; ++rho) {
       e[rho] = pe[rho * st];
       o[rho] = po[rho * st];
+    }
+    if (M > h) {  // block-uniform; bin a also takes (-1)^s conj g_{n-a}
+      const typename X::R sg = rp.s ? -1 : 1;
+#pragma unroll
+      for (int h8 = 0; h8 < 16; h8 += 8) {
+        C ec[8], oc[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int m = n - (j + T * (h8 + q));
+          const int64_t mc = m <= M ? m : M;
+          ec[q] = qe[mc * qs];
+          oc[q] = qo[mc * qs];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          if (n - (j + T * (h8 + q)) > M) continue;
+          e[h8 + q].x = fma(sg, ec[q].x, e[h8 + q].x);
+          e[h8 + q].y = fma(-sg, ec[q].y, e[h8 + q].y);
+          o[h8 + q].x = fma(sg, oc[q].x, o[h8 + q].x);
+          o[h8 + q].y = fma(-sg, oc[q].y, o[h8 + q].y);
+        }
+      }
     }
 #pragma unroll
     for (int rho = 0; rho < 16; ++rho) {
@@ -271,7 +309,7 @@ __device__ __forceinline__ void belt_pair(const RingPair &rp, const C *__restric
 #pragma unroll
     for (int rho = 0; rho < 16; ++rho) bufs[pad(j + T * rho)] = xs[rho];
     if (j == 0) bufs[pad(h)] = xsh;
-    __syncthreads();
+    fft16::job_sync<belt_nt<P, C>()>();
     C v[2][16];
     {
       const double2 ostep = expipi(2 * T, n);
@@ -284,20 +322,20 @@ __device__ __forceinline__ void belt_pair(const RingPair &rp, const C *__restric
         om = cmul(om, ostep);
       }
     }
-    fft16::fft2<P, true>(v, buf, bufs, twl, j);
+    fft16::fft2<P, true, belt_nt<P, C>()>(v, buf, bufs, twl, j);
     if (act) put16<T>(outn, j, v[0], K);
     if (act && south) put16<T>(outs, j, v[1], K);
     return;
   }
-  __syncthreads();
+  fft16::job_sync<belt_nt<P, C>()>();
   // 2. northern ring
   belt_fft_out<P>(buf, twl, j, n, act, K, outn);
   // 3. southern ring: X^S through the same buffer
-  __syncthreads();  // last FFT pass reads done
+  fft16::job_sync<belt_nt<P, C>()>();  // last FFT pass reads done
 #pragma unroll
   for (int rho = 0; rho < 16; ++rho) buf[pad(j + T * rho)] = xs[rho];
   if (j == 0) buf[pad(h)] = xsh;
-  __syncthreads();
+  fft16::job_sync<belt_nt<P, C>()>();
   asm volatile("" : "+v"(j));  // no address of the northern pass kept live
   belt_fft_out<P>(buf, twl, j, n, act && south, K, outs);
 }
@@ -468,7 +506,7 @@ __device__ __forceinline__ void belt_block_maps2(const LegTables &t, const RingT
   for (int ring = 0; ring < 2; ++ring) {
     if (ring == 1) {
       // southern ring: X^S of both maps through the same buffers
-      __syncthreads();  // last FFT pass reads done
+      fft16::job_sync<belt_nt<P, C>()>();  // last FFT pass reads done
 #pragma unroll
       for (int rho = 0; rho < 16; ++rho) {
         buf0[pad(j + T * rho)] = xs0[rho];
@@ -479,7 +517,7 @@ __device__ __forceinline__ void belt_block_maps2(const LegTables &t, const RingT
         buf1[pad(h)] = xsh1;
       }
     }
-    __syncthreads();
+    fft16::job_sync<belt_nt<P, C>()>();
     C v[2][16];
     {
       const double2 ostep = expipi(2 * T, n);
@@ -492,7 +530,7 @@ __device__ __forceinline__ void belt_block_maps2(const LegTables &t, const RingT
         om = cmul(om, ostep);
       }
     }
-    fft16::fft2<P, true>(v, buf0, buf1, twl, j);
+    fft16::fft2<P, true, belt_nt<P, C>()>(v, buf0, buf1, twl, j);
     if (act && (ring == 0 || south)) put16x2<T>(ring ? outs : outn, j, v[0], v[1], K, two);
   }
 }
@@ -510,7 +548,7 @@ __device__ __forceinline__ void belt_block(const LegTables &t, const RingTables 
     }
   }
   int jb, j;
-  job_lane<T>(threadIdx.x, &jb, &j);
+  job_lane<T>(job_tid<belt_nt<P, C>()>(), &jb, &j);
   C *buf = lds + jb * S * ring16_bufs(kRingBelt16, P, sizeof(C));
   int pi, k;
   const bool act = ring16_job(b, J, jb, t.K, count, &pi, &k);
@@ -613,9 +651,9 @@ __device__ __forceinline__ void wrap_fold2(const C *__restrict__ qe, const C *__
     if (rho < n) buf[pad(rho)] = on_n ? an[q] : X::mk(0.0, 0.0);
     if (!on_s) ps[q] = X::mk(0.0, 0.0);
   }
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
   wrap_fstep<P>(buf, n, s, tt, on_n ? g0n : X::mk(0.0, 0.0));
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
 }
 
 // The southern fold of wrap_fold2 into buf.  The caller has passed a
@@ -629,9 +667,9 @@ __device__ __forceinline__ void wrap_fold_south(C *buf, int n, int s, int tt, co
     const int rho = tt + T2 * q;
     if (rho < n) buf[pad(rho)] = ps[q];
   }
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
   wrap_fstep<P>(buf, n, s, tt, g0s);
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
 }
 
 // Fold of a cap ring pair without wrap (n > mmax): F_b = g_b
@@ -676,7 +714,7 @@ __device__ __forceinline__ void cap_fold2(const C *__restrict__ qe, const C *__r
     cn[rho] = (on_n && dm) ? cc : X::mk(0.0, 0.0);
     cs[rho] = (on_s && dm) ? dd : X::mk(0.0, 0.0);
   }
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
 #pragma unroll
   for (int rho = 0; rho < 8; ++rho) {
     const int m = h + tt + T2 * rho;
@@ -687,7 +725,7 @@ __device__ __forceinline__ void cap_fold2(const C *__restrict__ qe, const C *__r
       fs = cadd(fs, cs[rho]);
     }
   }
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
 }
 
 // Z entries of one cap ring from its fold F[0 .. h] in bufF: entry
@@ -740,14 +778,14 @@ __device__ __forceinline__ void cap_xform(const RingPair &rp, int K,
   }
   // Bluestein: y = IFFT(vhat . FFT(c . Z)) in the half's own buffer
   C *buf = half ? bufB : bufA;
-  fft16::fft<P, false>(v, buf, twl, j);
+  fft16::fft<P, false, cap_nt<P, C>()>(v, buf, twl, j);
   asm volatile("" : "+v"(tt));
 #pragma unroll
   for (int rho = 0; rho < 16; ++rho) v[rho] = cmul(v[rho], X::of(vhat[j + T * rho]));
-  fft16::fft<P, true>(v, buf, twl, j);
+  fft16::fft<P, true, cap_nt<P, C>()>(v, buf, twl, j);
   asm volatile("" : "+v"(tt));
   // A_p = c_p y_p into bufA, e^{2 pi i p/h} c_p y_p (B) into bufB, p < i
-  __syncthreads();  // last-pass reads of buf done
+  fft16::job_sync<cap_nt<P, C>()>();  // last-pass reads of buf done
   {
     const double2 ostep = expipi(4 * T, n);
     double2 om = half ? expipi(4 * j, n) : make_double2(1.0, 0.0);
@@ -759,7 +797,7 @@ __device__ __forceinline__ void cap_xform(const RingPair &rp, int K,
       om = cmul(om, st);
     }
   }
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
   // z_p = A_p + B_p, z_{p+i} = A_p - B_p
   if (on) {
 #pragma unroll
@@ -798,7 +836,7 @@ __device__ __forceinline__ void cap_xform2(const RingPair &rp, int K,
     v[0][8 + rho] = v[1][8 + rho] = X::mk(0.0, 0.0);
   }
   C *b0 = half ? BN : AN, *b1 = half ? BS : AS;
-  fft16::fft2<P, false>(v, b0, b1, twl, j);
+  fft16::fft2<P, false, cap_nt<P, C>()>(v, b0, b1, twl, j);
   asm volatile("" : "+v"(tt));
 #pragma unroll
   for (int rho = 0; rho < 16; ++rho) {
@@ -806,9 +844,9 @@ __device__ __forceinline__ void cap_xform2(const RingPair &rp, int K,
     v[0][rho] = cmul(v[0][rho], vh);
     v[1][rho] = cmul(v[1][rho], vh);
   }
-  fft16::fft2<P, true>(v, b0, b1, twl, j);
+  fft16::fft2<P, true, cap_nt<P, C>()>(v, b0, b1, twl, j);
   asm volatile("" : "+v"(tt));
-  __syncthreads();  // last-pass reads of the buffers done
+  fft16::job_sync<cap_nt<P, C>()>();  // last-pass reads of the buffers done
   {
     const double2 ostep = expipi(4 * T, n);
     double2 om = half ? expipi(4 * j, n) : make_double2(1.0, 0.0);
@@ -824,7 +862,7 @@ __device__ __forceinline__ void cap_xform2(const RingPair &rp, int K,
       om = cmul(om, st);
     }
   }
-  __syncthreads();
+  fft16::job_sync<cap_nt<P, C>()>();
   if (!own) return;
 #pragma unroll
   for (int rho = 0; rho < 4; ++rho) {
@@ -950,7 +988,7 @@ __device__ __forceinline__ void cap_block_maps2(const LegTables &t, const RingTa
   for (int ring = 0; ring < 2; ++ring) {
     if (ring == 1) {
       if (!south) break;  // block-uniform
-      __syncthreads();    // pixel reads of the northern ring done
+      fft16::job_sync<cap_nt<P, C>()>();    // pixel reads of the northern ring done
     }
     C za[8], zb[8];
     if (ring == 0 || !park) {
@@ -981,7 +1019,7 @@ __device__ __forceinline__ void cap_block_maps2(const LegTables &t, const RingTa
         zb[e] = cx<C>::mk(b.x, b.y);
       }
     }
-    __syncthreads();  // fold reads done before the transforms write the buffers
+    fft16::job_sync<cap_nt<P, C>()>();  // fold reads done before the transforms write the buffers
     asm volatile("" : "+v"(tt));
     cap_xform2<P>(rp, K, chirp, vhat, za, zb, b0, b1, b2, b3, twl, tt, false, false, false,
                   nullptr, nullptr);
@@ -1253,8 +1291,9 @@ __device__ __forceinline__ void cap_block(const LegTables &t, const RingTables &
       return;
     }
   }
-  const int jb = threadIdx.x / (2 * T);
-  int tt = threadIdx.x % (2 * T);
+  const int tid = job_tid<cap_nt<P, C>()>();
+  const int jb = tid / (2 * T);
+  int tt = tid % (2 * T);
   C *bufA = lds + ring16_bufs(kRingCap16, P, sizeof(C)) * jb * S, *bufB = bufA + S;
   C *bufA2 = bufB + S, *bufB2 = bufA2 + S;  // dual only
   int pi, k;
@@ -1295,7 +1334,7 @@ __device__ __forceinline__ void cap_block(const LegTables &t, const RingTables &
     C ps[16], g0s;
     wrap_fold2<P>(qe, qo, qs, M, rp.n, rp.s, bufA, tt, act, act && south, ps, &g0s);
     cap_z<P>(rp, chirp, bufA, tt, zn);
-    __syncthreads();  // reads of the northern fold done
+    fft16::job_sync<cap_nt<P, C>()>();  // reads of the northern fold done
     wrap_fold_south<P>(bufA, rp.n, rp.s, tt, ps, g0s);
     cap_z<P>(rp, chirp, bufA, tt, zs);
   } else {
@@ -1305,7 +1344,7 @@ __device__ __forceinline__ void cap_block(const LegTables &t, const RingTables &
   }
   asm volatile("" : "+v"(tt));  // no table load hoisted above the barriers
   cap_xform<P>(rp, K, chirp, vhat, zn, bufA, bufB, twl, tt, act, map + k + rp.pix_n * K);
-  __syncthreads();  // the northern ring's reads of bufA / bufB done
+  fft16::job_sync<cap_nt<P, C>()>();  // the northern ring's reads of bufA / bufB done
   asm volatile("" : "+v"(tt));
   cap_xform<P>(rp, K, chirp, vhat, zs, bufA, bufB, twl, tt, act && south,
                map + k + (south ? rp.pix_s : 0) * K);
@@ -1353,6 +1392,97 @@ __global__ __launch_bounds__(ring16_threads(KIND, P, sizeof(C)),
   ring16_block<KIND, P>(t, rt, first, count, map, blockIdx.x, (C *)(lds + kTwSlots), twl);
 }
 
+// Transforms of up to kSmallP points take one launch for all their launch
+// groups (FP64): the groups of a small map are a few blocks each, and one
+// after the other they cost a launch gap and the latency of a whole block
+// each.  Workgroups of 128 threads run a block of a 128-thread class or, side
+// by side and without common barriers, two of a one-wave class.  Measured, us
+// of the
+// ring stage, a launch per group / this: Nside 64, 1 map 43 / 28; Nside 300, 5
+// maps 185 / 132; Nside 512, 1 map 71 / 49; 64 maps at Nside 1024 no change.
+constexpr int kSmallP = 1024;
+constexpr int kSmallThreads = 128;
+struct SmallGroups {
+  int n = 0;
+  int g[kMaxLaunches], end[kMaxLaunches];  // launch group, end of its workgroups
+};
+
+template <int KIND, int P>
+constexpr size_t small_bytes() {
+  return (size_t)kTwSlots * sizeof(double2) +
+         (kSmallThreads / ring16_threads(KIND, P, sizeof(double2))) *
+             (ring16_bytes(KIND, P, sizeof(double2)) - kTwSlots * sizeof(double2));
+}
+
+template <int KIND, int P>
+__device__ __forceinline__ void small_block(const LegTables &t, const RingTables &rt, int g,
+                                            double *__restrict__ map, int b, double2 *lds,
+                                            const double2 *twl) {
+  constexpr int NT = ring16_threads(KIND, P, sizeof(double2));
+  static_assert(NT == 64 || NT == kSmallThreads, "one or two blocks per workgroup");
+  if constexpr (NT == 64) {
+    // two virtual blocks on this workgroup's XCD, consecutive there
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    b = ((b >> 3) * 2 + wv) * 8 + (b & 7);
+    lds += wv * ring16_bufs(KIND, P, sizeof(double2)) * ring16_jobs(KIND, P, sizeof(double2)) *
+           job_slots(P);
+  }
+  ring16_block<KIND, P>(t, rt, rt.first[g], rt.count[g], map, b, lds, twl);
+}
+
+#define WM_SMALL_SIZES(X) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
+
+__global__ __launch_bounds__(kSmallThreads, 2) void k_ring16_small(LegTables t, RingTables rt,
+                                                                   SmallGroups sg,
+                                                                   double *__restrict__ map) {
+  extern __shared__ double2 lds[];
+  double2 *twl = lds;
+  load_twiddles16<kSmallThreads>(twl, rt.twiddle);
+  __syncthreads();
+  int i = 0, b = blockIdx.x;
+  while (b >= sg.end[i]) ++i;
+  if (i > 0) b -= sg.end[i - 1];
+  const int g = sg.g[i];
+  switch (rt.kind[g] * 16384 + rt.fftP[g]) {
+#define WM_SMALL_K(KIND, P) \
+  case KIND * 16384 + P: small_block<KIND, P>(t, rt, g, map, b, lds + kTwSlots, twl); break;
+#define WM_SMALL(P) WM_SMALL_K(kRingBelt16, P) WM_SMALL_K(kRingCap16, P) WM_SMALL_K(kRingWrap16, P)
+    WM_SMALL_SIZES(WM_SMALL)
+#undef WM_SMALL
+#undef WM_SMALL_K
+  }
+}
+
+bool ring16_small(int kind, int P) { return kind != kRingGeneral && kind != kRingLong && P <= kSmallP; }
+
+// Every launch group of rt that ring16_small takes, in one launch (FP64 q).
+hipError_t launch_ring16_small(const LegTables &t, const RingTables &rt, double *map,
+                               hipStream_t s) {
+  SmallGroups sg;
+  size_t lds = 0;
+  int64_t total = 0;
+  for (int g = 0; g < rt.nlaunch; ++g) {
+    if (rt.count[g] == 0 || !ring16_small(rt.kind[g], rt.fftP[g])) continue;
+    const int64_t nb = ring16_blocks(rt.kind[g], rt.fftP[g], t.K, rt.count[g], sizeof(double2));
+    const int per = kSmallThreads / ring16_threads(rt.kind[g], rt.fftP[g], sizeof(double2));
+    total += (nb / 8 + per - 1) / per * 8;
+    sg.g[sg.n] = g;
+    sg.end[sg.n++] = (int)total;
+#define WM_SMALL_K(KIND, P)                            \
+  if (rt.kind[g] == KIND && rt.fftP[g] == P)           \
+    lds = lds < small_bytes<KIND, P>() ? small_bytes<KIND, P>() : lds;
+#define WM_SMALL(P) WM_SMALL_K(kRingBelt16, P) WM_SMALL_K(kRingCap16, P) WM_SMALL_K(kRingWrap16, P)
+    WM_SMALL_SIZES(WM_SMALL)
+#undef WM_SMALL
+#undef WM_SMALL_K
+  }
+  if (sg.n == 0) return hipSuccess;
+  if (total > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_ring16_small, dim3((unsigned)total), dim3(kSmallThreads), lds, s, t, rt, sg,
+                     map);
+  return hipGetLastError();
+}
+
 // Ring kernel of a batch: block i runs item r16items[first + i] (request,
 // launch group, block) as the single-plan kernel runs block b (bitwise the
 // same maps).  One item per block, in the host's order, rather than a
@@ -1377,27 +1507,54 @@ __global__ __launch_bounds__(ring16_threads(KIND, P, sizeof(double2)),
 
 bool ring16_size_ok(int P) { return P >= 16 && P <= 8192 && (P & (P - 1)) == 0; }
 
+template <int KIND, int P>
+static hipError_t set_lds_limit() {
+  const auto set = [](const void *f, size_t bytes) {
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  };
+  hipError_t e = set((const void *)k_batch_ring16<KIND, P>, ring16_bytes(KIND, P, sizeof(double2)));
+  if (e == hipSuccess)
+    e = set((const void *)k_ring16<KIND, P, float2>, ring16_bytes(KIND, P, sizeof(float2)));
+  if constexpr (P > kSmallP) {
+    if (e == hipSuccess)
+      e = set((const void *)k_ring16<KIND, P, double2>, ring16_bytes(KIND, P, sizeof(double2)));
+  }
+  return e;
+}
+
 hipError_t ring16_set_lds_limits() {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
-#define WM_SET_K(KIND, P)                                                                  \
-  for (const void *f : {(const void *)k_ring16<KIND, P, double2>,                          \
-                        (const void *)k_batch_ring16<KIND, P>})                            \
-    if (err == hipSuccess)                                                                 \
-      err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,             \
-                                (int)ring16_bytes(KIND, P, sizeof(double2)));              \
-  if (err == hipSuccess)                                                                   \
-    err = hipFuncSetAttribute((const void *)k_ring16<KIND, P, float2>,                     \
-                              hipFuncAttributeMaxDynamicSharedMemorySize,                  \
-                              (int)ring16_bytes(KIND, P, sizeof(float2)));
-#define WM_SET(P) WM_SET_K(kRingBelt16, P) WM_SET_K(kRingCap16, P) WM_SET_K(kRingWrap16, P)
+    size_t small = 0;
+#define WM_SMALL(P)                                                                        \
+  for (size_t v : {small_bytes<kRingBelt16, P>(), small_bytes<kRingCap16, P>(),            \
+                   small_bytes<kRingWrap16, P>()})                                         \
+    if (v > small) small = v;
+    WM_SMALL_SIZES(WM_SMALL)
+#undef WM_SMALL
+    err = hipFuncSetAttribute((const void *)k_ring16_small,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)small);
+#define WM_SET(P)                                                       \
+  if (err == hipSuccess) err = set_lds_limit<kRingBelt16, P>();         \
+  if (err == hipSuccess) err = set_lds_limit<kRingCap16, P>();          \
+  if (err == hipSuccess) err = set_lds_limit<kRingWrap16, P>();
     WM_RING16_SIZES(WM_SET)
 #undef WM_SET
-
-#undef WM_SET_K
   });
   return err;
+}
+
+template <int KIND, int P>
+static hipError_t launch_fp64(const LegTables &t, const RingTables &rt, int first, int count,
+                              double *map, int64_t nb, dim3 nthr, size_t lds, hipStream_t s) {
+  if constexpr (P > kSmallP) {
+    hipLaunchKernelGGL((k_ring16<KIND, P, double2>), dim3((unsigned)nb), nthr, lds, s, t, rt,
+                       first, count, map);
+    return hipGetLastError();
+  } else {
+    return hipErrorInvalidValue;  // launch_ring16_small takes these
+  }
 }
 
 // pairs order[first .. first + count) of one launch group (kind, FFT size
@@ -1416,11 +1573,10 @@ hipError_t launch_ring16(int kind, int P, const LegTables &t, const RingTables &
 #define WM_CASE_K(KIND, PP)                                                                \
   if (kind == KIND && P == PP) {                                                           \
     if (t.q32)                                                                             \
-      hipLaunchKernelGGL((k_ring16<KIND, PP, float2>), dim3((unsigned)nb), nthr, lds,  \
-                         s, t, rt, first, count, map);                                     \
+      hipLaunchKernelGGL((k_ring16<KIND, PP, float2>), dim3((unsigned)nb), nthr, lds, s, t, \
+                         rt, first, count, map);                                           \
     else                                                                                   \
-      hipLaunchKernelGGL((k_ring16<KIND, PP, double2>), dim3((unsigned)nb), nthr, lds, \
-                         s, t, rt, first, count, map);                                     \
+      return launch_fp64<KIND, PP>(t, rt, first, count, map, nb, nthr, lds, s);            \
     return hipGetLastError();                                                              \
   }
 #define WM_CASE(PP) WM_CASE_K(kRingBelt16, PP) WM_CASE_K(kRingCap16, PP) WM_CASE_K(kRingWrap16, PP)

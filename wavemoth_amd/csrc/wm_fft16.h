@@ -13,8 +13,8 @@
 // canonical layout and the last pass (Ns R = P) writes it, so a forward
 // transform, a pointwise product and an inverse transform chain in
 // registers.  Every pass but the last costs one LDS round trip and two
-// barriers; the barriers are block-wide, so all jobs of a block run the
-// same pass sequence.
+// barriers; the barriers are block-wide (wave-wide for jobs that share a
+// wave), so all jobs of a block run the same pass sequence.
 #pragma once
 
 #include "wm_fft.h"
@@ -33,6 +33,18 @@ constexpr int kThreads = 256;  // threads per block of the register-FFT kernels
 __host__ __device__ constexpr int pad(int d) { return d + (d >> 4); }
 // LDS slots of one job's buffer for an FFT of P points plus one extra bin
 __host__ __device__ constexpr int job_slots(int P) { return pad(P) + 2; }
+
+// Barrier of the NT threads that share jobs: within a wave, in program order.
+template <int NT>
+__device__ __forceinline__ void job_sync() {
+  if constexpr (NT <= 64) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
 
 // 16-point DFT in registers, y_k = sum_r v_r e^{-/+ 2 pi i r k/16} (INV: +).
 // Radix 4 x 4: r = r0 + 4 r1, k = k1 + 4 k2; y_k ends in v[4 (k & 3) + (k >> 2)].
@@ -87,7 +99,7 @@ __device__ __forceinline__ void dft_r(C *x) {
 // thread layout: transform t in v[t] with LDS buffer buf[t]; twl the
 // two-level twiddle table, j the thread's index in its job.  The twiddle
 // powers are formed once for all NV transforms.
-template <int P, int Ns, bool INV, int NV, typename C>
+template <int P, int Ns, bool INV, int NV, int NT, typename C>
 __device__ __forceinline__ void pass(C (&v)[NV][16], C *const (&buf)[NV], const double2 *twl,
                                      int j) {
   constexpr int T = P / 16;
@@ -134,7 +146,7 @@ __device__ __forceinline__ void pass(C (&v)[NV][16], C *const (&buf)[NV], const 
 #pragma unroll
         for (int r = 0; r < R; ++r) v[t][q + Q * r] = x[t][q][r];
   } else {
-    __syncthreads();  // every read of buf (this pass or earlier users) done
+    job_sync<NT>();  // every read of buf (this pass or earlier users) done
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int jq = j + T * q;
@@ -145,8 +157,8 @@ __device__ __forceinline__ void pass(C (&v)[NV][16], C *const (&buf)[NV], const 
 #pragma unroll
         for (int r = 0; r < R; ++r) buf[t][pad(d + Ns * r)] = x[t][q][r];
     }
-    __syncthreads();
-    pass<P, Ns * R, INV, NV>(v, buf, twl, j);
+    job_sync<NT>();
+    pass<P, Ns * R, INV, NV, NT>(v, buf, twl, j);
   }
 }
 
@@ -154,23 +166,24 @@ __device__ __forceinline__ void pass(C (&v)[NV][16], C *const (&buf)[NV], const 
 // layout, in place: INV = false e^{-2 pi i jk/P}, INV = true e^{+...};
 // unnormalised.  Starts with a barrier before its first LDS write, so
 // the caller may still read buf up to the call.  Every thread of the
-// block must call it.
-template <int P, bool INV, typename C>
+// block must call it, or of the wave where NT, the threads that share jobs
+// and meet at its barriers, is 64.
+template <int P, bool INV, int NT = 1024, typename C>
 __device__ __forceinline__ void fft(C v[16], C *buf, const double2 *twl, int j) {
   static_assert(P >= 16 && P <= kMaxFFT && (P & (P - 1)) == 0, "P");
   C(&vv)[1][16] = *reinterpret_cast<C(*)[1][16]>(v);
   C *const bb[1] = {buf};
-  pass<P, 1, INV, 1>(vv, bb, twl, j);
+  pass<P, 1, INV, 1, NT>(vv, bb, twl, j);
 }
 
 // Two independent transforms of the same size and direction together
 // (buffers buf0, buf1): half the barriers of two calls of fft.
-template <int P, bool INV, typename C>
+template <int P, bool INV, int NT = 1024, typename C>
 __device__ __forceinline__ void fft2(C (&v)[2][16], C *buf0, C *buf1, const double2 *twl,
                                      int j) {
   static_assert(P >= 16 && P <= kMaxFFT && (P & (P - 1)) == 0, "P");
   C *const bb[2] = {buf0, buf1};
-  pass<P, 1, INV, 2>(v, bb, twl, j);
+  pass<P, 1, INV, 2, NT>(v, bb, twl, j);
 }
 
 }  // namespace fft16

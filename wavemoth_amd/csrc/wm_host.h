@@ -125,8 +125,9 @@ hipError_t launch_long_bluestein_prep(const double2 *twiddle, double2 *chirp, do
 
 // Ring geometry, Bluestein tables and the single-transform launch groups.
 // wide: plan for kRingWideMaps or more maps (wrapping rings then take the
-// register-FFT kernel, which needs many maps to fill the device).
+// register-FFT kernel, which needs many maps to fill the device).  fp64: an
+// FP64 plan's, whose belt kernel also takes power-of-two rings with mmax < n.
 bool build_ring_geometry(DevArena &a, RingTables &rt, RingHost &host, int N, int M,
-                         bool phase_shifts, bool wide, hipStream_t s);
+                         bool phase_shifts, bool wide, bool fp64, hipStream_t s);
 
 }  // namespace wm

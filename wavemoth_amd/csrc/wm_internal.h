@@ -306,6 +306,10 @@ int64_t ring16_blocks(int kind, int P, int K, int count, int cs);
 hipError_t ring16_set_lds_limits();
 hipError_t launch_ring16(int kind, int P, const LegTables &t, const RingTables &rt, int first,
                          int count, double *map, hipStream_t s);
+// The FP64 groups of short transforms, all in one launch.
+bool ring16_small(int kind, int P);
+hipError_t launch_ring16_small(const LegTables &t, const RingTables &rt, double *map,
+                               hipStream_t s);
 hipError_t launch_batch_ring16(int kind, int P, const BatchDev &d, int first, int count,
                                hipStream_t s);
 int adjoint_groups(const LegTables &t);
