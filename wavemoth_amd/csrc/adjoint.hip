@@ -17,9 +17,10 @@
 //     bins past n/2), then q_even = F_north + F_south, q_odd = F_north -
 //     F_south (the equator ring feeds both), into the [R][2][M+1][K] buffer.
 //  2. k_legendre_adj: b~_l = sum_rings L~_l(x_r) q_{parity(l-m)}(r) with the
-//     same monic recurrence, seeds and l-segments as the synthesis, the sum
-//     over rings on the matrix cores.
+//     same recurrences, seeds and l-segments as the synthesis, the sum over
+//     rings on the matrix cores.
 //  3. k_adj_finish: b_lm = c_m A_l sum_groups b~ into the m-major layout.
+#include <cmath>
 #include <mutex>
 
 #include "wm_fft16.h"
@@ -387,46 +388,43 @@ __device__ __forceinline__ double lane_xor8(double x) { return dpp_move<0x128>(x
 __device__ __forceinline__ double lane_xor4(double x) { return dpp_move<0x1b>(dpp_move<0x141>(x)); }
 
 // b~ partial sums on the FP64 matrix cores.  A wave is one work item (m, ring
-// group g): units of 16 GR rings c = g, g + G, ... one after the other, for
-// each the whole l-range of the unit's rings in four segments, as in the
-// matrix-core synthesis sweep (the same segments and checkpoints).  Lane
-// 4 i + u steps segment u of ring i of every 16-ring group: with A[row][k]
-// on lane row + 4 block + 16 k that is a product, in each of the 4 blocks of
-// v_mfma_f64_4x4x4f64, of 4 l (one per segment) with 4 rings as it stands,
-// and B, 4 columns (the real and imaginary parts of 2 maps, of the step's
-// parity), has q of the same ring on lane 4 i + column: 16 distinct rings in
-// 64 lanes, so that one unit's q of both parities stays in 4 GR registers per
-// 2 maps.  The GR products of a step add up in one accumulator; the 4 blocks
-// of 4 steps are then summed by two exchange-and-add stages that leave step b
-// in block b, one row of 4 columns per lane quad.
+// group g): units of 16 GR rings one after the other, for each the whole
+// l-range of the unit's rings in four segments, as in the matrix-core
+// synthesis sweep (the same segments and checkpoints).  Lane 4 i + u steps
+// segment u of ring i of every 16-ring group: with A[row][k] on lane row +
+// 4 block + 16 k that is a product, in each of the 4 blocks of
+// v_mfma_f64_4x4x4f64, of 4 l (one per segment) with 4 rings as it stands, and
+// B has q of the same ring on lane 4 i + column: 16 distinct rings in 64 lanes.
+// The GR products of a step add up in one accumulator; the 4 blocks of 4
+// steps are then summed by two exchange-and-add stages that leave step b in
+// block b, one row of 4 columns per lane quad.
 //
-// FP64 matrix and vector instructions share one pipe, so a step costs GR (2
-// FP64 + CG products of 16 cycles): at one map half of the 4 columns are
-// empty, where the 16 x 16 form of one row parity per column half (before)
-// left 14 of 16 empty: Nside 2048, lmax 4096, 1 map 19.0 -> 6.2 ms; Nside
-// 512, 3 maps 0.427 -> 0.28 ms.
-template <int CG, int GR>
-__global__ __launch_bounds__(64, CG == 1 ? 3 : 2) void k_legendre_adj(LegTables t, int G, int kb, int kn,
-                                                     double2 *partial) {
-  constexpr int ST = 4, RU = 16 * GR;
-  __shared__ double2 seeds[RU];  // of the unit's rings: a load where one joins would stall
-  const int lane = threadIdx.x;
+// FP64 matrix and vector instructions share one pipe, and a product takes four
+// times a vector instruction.  Units in the middle latitudes run in the pair
+// form (legendre.hip): a step of two l costs 2 vector instructions and one
+// product per map, whose 4 columns are the real and imaginary parts of the
+// even and, times x, the odd sums.  The other units step l by l: 2 vector
+// instructions and, for every 2 maps, one product of which one parity's
+// columns are wanted; per two l and 16 rings 4 + 8 against 2 + 4 instruction
+// times at 1 map, 4 + 16 against 2 + 12 at 3.  A group's units are all of one
+// form: its rows of partial sums are b~_l or the sums of p_k.
+// The units c = c0, c0 + step, ... of `units` one-step units (those below ua,
+// then those from ub on).
+template <int KN, int GR>
+__device__ __forceinline__ void adj_units(const LegTables &t, int c0, int step, int units, int ua,
+                                          int ub, int m, int kb, double *prow, int lane,
+                                          double2 *seeds) {
+  constexpr int ST = 4, RU = 16 * GR, CG = (KN + 1) / 2, kn = KN;
   const int L = t.L, R = t.R, M = t.M, K = t.K;
-  // block b runs on XCD b % 8; runs of 8 consecutive m share an XCD, since 8
-  // entries of q (at one map) share a line
-  const int xi = blockIdx.x >> 3, g = xi % G, mi = xi / G;
-  const int m = ((mi >> 3) * 8 + (blockIdx.x & 7)) * 8 + (mi & 7);
-  if (m > M) return;
   const int u = lane & 3, ring = lane >> 2;  // segment (and column of B), ring in a group
   const int b = ring & 3, ds = lane >> 4;    // block, segment of the result rows
   const int64_t offm = t.off[m];
   const double *ct0 = t.ctil + (offm - m);
   const double *cs0 = t.cscale + offm / kChunk;
-  double *prow = (double *)(partial + ((int64_t)g * t.nlpad + offm) * K + kb);
   const unsigned rstride = 2 * (unsigned)K;  // doubles per l row of the partial sums
-  const int units = (R + RU - 1) / RU;
   bool first = true;
-  for (int c = g; c < units; c += G) {
+  for (int ci = c0; ci < units; ci += step) {
+    const int c = ci < ua ? ci : ci - ua + ub;
     const int l0 = __builtin_amdgcn_readfirstlane(
         t.seg_l0[(int64_t)m * t.SW + c * RU / kSegRings]);
     if (l0 > L) continue;
@@ -570,10 +568,191 @@ __global__ __launch_bounds__(64, CG == 1 ? 3 : 2) void k_legendre_adj(LegTables 
     }
 }
 
-// b_lm = c_m A_l sum_g partial[g], into the m-major complex layout; one
-// thread per (row, map), so that each group's partial sums are read
-// contiguously across the threads.
-__global__ __launch_bounds__(256) void k_adj_finish(LegTables t, int G,
+
+// The pair-form units c = c0, c0 + step, ... < ub: row k of the partial sums
+// takes the places of the rows l = m + 2 k (sums of p_k q_even) and l + 1
+// (p_k x q_odd).  Seeds and checkpoints are the one-step form's, converted.
+template <int KN, int GR>
+__device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int step, int ub, int m,
+                                               int kb, double *prow, int lane, double2 *seeds) {
+  constexpr int ST = 4, RU = 16 * GR, KC = kChunk / 2;  // steps of a chunk
+  const int L = t.L, M = t.M, K = t.K;
+  const int u = lane & 3, ring = lane >> 2;  // segment (and column of B), ring in a group
+  const int b = ring & 3, ds = lane >> 4;    // block, segment of the result rows
+  const int64_t offm = t.off[m];
+  const double *ct0 = t.ctil + (offm - m);
+  const double2 *h0 = t.pair_h + offm / kChunk;
+  const unsigned rstride = 2 * (unsigned)K;  // doubles per l row of the partial sums
+  bool first = true;
+  for (int c = c0; c < ub; c += step) {
+    const int l0 = __builtin_amdgcn_readfirstlane(
+        t.seg_l0[(int64_t)m * t.SW + c * RU / kSegRings]);
+    if (l0 > L) continue;
+    if (first) {  // rows no unit has written yet
+      for (int j = lane; j < (l0 - m) * 2 * KN; j += 64) {
+        const int l = j / (2 * KN);
+        prow[(int64_t)l * rstride + (j - l * 2 * KN)] = 0.0;
+      }
+    }
+    const int nc = (L - l0) / kChunk + 1, ns = (nc + 3) / 4;
+    const int cb = u * ns;
+    // (L~_{l-1}, L~_l) at the start of a chunk -> (p_{k-1}, p_k)
+    auto to_pair = [&](double2 v, double x, int l) {
+      const double2 h = h0[(l - m) / kChunk];
+      const double rx = 1.0 / x;
+      return make_double2(v.x * h.y * rx, fma(x, v.y, -(ct0[l] * v.x)) * h.x * rx);
+    };
+#pragma unroll
+    for (int i = 0; i < RU / 64; ++i) {
+      const int r = c * RU + 64 * i + lane;
+      const int s = t.seed_l[(int64_t)m * t.R + r];
+      if (s <= L) seeds[64 * i + lane] = to_pair(t.seed_v[(int64_t)m * t.R + r], t.ring_x[r], s);
+    }
+    const bool polar = t.ring_x[c * RU] > 0.7;  // wave-uniform
+    double y[GR], prev[GR], cur[GR], bq[KN][GR];
+    int sl[GR];
+#pragma unroll
+    for (int i = 0; i < GR; ++i) {
+      const int r = c * RU + 16 * i + ring;
+      const double x = t.ring_x[r];
+      y[i] = polar ? -fma(-x, x, 1.0) : x * x;
+      sl[i] = t.seed_l[(int64_t)m * t.R + r];
+      double2 v = make_double2(0.0, 0.0);
+      if (u > 0 && cb < nc)
+        v = to_pair(t.ckpt[((int64_t)m * 3 + u - 1) * t.R + r], x, l0 + kChunk * cb);
+      prev[i] = v.x;
+      cur[i] = v.y;
+#pragma unroll
+      for (int k = 0; k < KN; ++k) {
+        const double q =
+            ((const double *)t.qbuf)[2 * q_index(r, u >> 1, kb + k, m, K, M + 1) + (u & 1)];
+        bq[k][i] = u >= 2 ? q * x : q;
+      }
+    }
+    const double2 *pc = (polar ? t.pair_s : t.pair_x) + (offm + l0 - m) / 2;
+    double *pr = prow + (int64_t)(l0 - m + (u >> 1)) * rstride + (u & 1);
+    unsigned e = KC * (unsigned)(cb < nc ? cb : nc - 1);
+    double2 cc[ST];
+    double old[KN];
+#pragma unroll
+    for (int s = 0; s < ST; ++s) cc[s] = pc[e + s];
+    // row of the lane's results: segment ds, step b of a 4-step block; what
+    // earlier units left there is read one block ahead
+    const int drow0 = KC * ds * ns + b;
+    auto load_old = [&](int blk, double (&o)[KN]) {
+      const int dr = drow0 + ST * blk;
+      const bool rok = !first && ds * ns + blk / (KC / ST) < nc && l0 + 2 * dr <= L &&
+                       blk < ns * (KC / ST);
+#pragma unroll
+      for (int k = 0; k < KN; ++k) o[k] = rok ? pr[2 * (unsigned)dr * rstride + 2 * k] : 0.0;
+    };
+    wave_sync_lds();
+    load_old(0, old);
+    for (int j = 0; j < ns; ++j) {
+      const int ls = l0 + kChunk * (cb + j);
+      bool hit = false;
+#pragma unroll
+      for (int i = 0; i < GR; ++i) hit |= sl[i] == ls;
+      if (__any(hit)) {
+#pragma unroll
+        for (int i = 0; i < GR; ++i)
+          if (sl[i] == ls) {
+            const double2 v = seeds[16 * i + ring];
+            prev[i] = v.x;
+            cur[i] = v.y;
+          }
+      }
+      if (3 * ns + j >= nc && cb + j >= nc) {  // past the segment's rows
+#pragma unroll
+        for (int i = 0; i < GR; ++i) prev[i] = cur[i] = 0.0;
+      }
+      const unsigned en = KC * (unsigned)(cb + j + 1 < nc ? cb + j + 1 : nc - 1);
+      const int drow = drow0 + KC * j;
+      const bool dok = ds * ns + j < nc;
+#pragma unroll
+      for (int s0 = 0; s0 < KC; s0 += ST) {
+        double2 cn[ST];
+        double on[KN];
+#pragma unroll
+        for (int s = 0; s < ST; ++s) cn[s] = pc[(s0 + ST < KC ? e + s0 + ST : en) + s];
+        const bool rok = dok && l0 + 2 * (drow + s0) <= L;
+        const unsigned ro = 2 * (unsigned)(drow + s0) * rstride;
+        load_old(j * (KC / ST) + s0 / ST + 1, on);
+        __builtin_amdgcn_sched_barrier(0);
+        double d[ST][KN];
+#pragma unroll
+        for (int s = 0; s < ST; ++s)
+#pragma unroll
+          for (int k = 0; k < KN; ++k) d[s][k] = 0.0;
+        // two steps of a group at a time: their products go to two accumulators
+#pragma unroll
+        for (int s = 0; s < ST; s += 2)
+#pragma unroll
+          for (int i = 0; i < GR; ++i) {
+            const double nx = fma(fma(cc[s].x, y[i], cc[s].y), cur[i], -prev[i]);
+#pragma unroll
+            for (int k = 0; k < KN; ++k) {
+              d[s][k] = __builtin_amdgcn_mfma_f64_4x4x4f64(cur[i], bq[k][i], d[s][k], 0, 0, 0);
+              d[s + 1][k] =
+                  __builtin_amdgcn_mfma_f64_4x4x4f64(nx, bq[k][i], d[s + 1][k], 0, 0, 0);
+            }
+            prev[i] = nx;
+            cur[i] = fma(fma(cc[s + 1].x, y[i], cc[s + 1].y), nx, -cur[i]);
+          }
+#pragma unroll
+        for (int k = 0; k < KN; ++k) {
+          const bool b2 = b & 2, b1 = b & 1;
+          const double e0 = (b2 ? d[2][k] : d[0][k]) + lane_xor8(b2 ? d[0][k] : d[2][k]);
+          const double e1 = (b2 ? d[3][k] : d[1][k]) + lane_xor8(b2 ? d[1][k] : d[3][k]);
+          const double f = (b1 ? e1 : e0) + lane_xor4(b1 ? e0 : e1);
+          if (rok) pr[ro + 2 * k] = old[k] + f;
+        }
+#pragma unroll
+        for (int s = 0; s < ST; ++s) cc[s] = cn[s];
+#pragma unroll
+        for (int k = 0; k < KN; ++k) old[k] = on[k];
+      }
+      e = en;
+    }
+    // the next unit's segments give these rows to other lanes of the wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    first = false;
+  }
+  if (first)
+    for (int j = lane; j < (L - m + 1) * 2 * KN; j += 64) {
+      const int l = j / (2 * KN);
+      prow[(int64_t)l * rstride + (j - l * 2 * KN)] = 0.0;
+    }
+}
+
+// Groups g < G1 take the one-step units, the others the pair-form units.
+template <int KN, int GR>
+__global__ __launch_bounds__(64, KN <= 2 ? 3 : 2) void k_legendre_adj(LegTables t, int G, int G1,
+                                                                      int kb, double2 *partial) {
+  constexpr int RU = 16 * GR;
+  __shared__ double2 seeds[RU];  // of the unit's rings: a load where one joins would stall
+  // block b runs on XCD b % 8; runs of 8 consecutive m share an XCD, since 8
+  // entries of q (at one map) share a line
+  const int xi = blockIdx.x >> 3, g = xi % G, mi = xi / G;
+  const int m = ((mi >> 3) * 8 + (blockIdx.x & 7)) * 8 + (mi & 7);
+  if (m > t.M) return;
+  double *prow = (double *)(partial + ((int64_t)g * t.nlpad + t.off[m]) * t.K + kb);
+  const int all = (t.R + RU - 1) / RU;
+  int ua = all, ub = all;
+  if (G1 < G) pair_units(t, RU, &ua, &ub);
+  if (g < G1)
+    adj_units<KN, GR>(t, g, G1, all - (ub - ua), ua, ub, m, kb, prow, threadIdx.x, seeds);
+  else
+    adj_pair_units<KN, GR>(t, ua + g - G1, G - G1, ub, m, kb, prow, threadIdx.x, seeds);
+}
+
+// b_lm = c_m sum_g, from b~ (times A_l) of the one-step groups and from the
+// sums S_k of the pair-form groups: Lambda_{l+1} = x P_k, Lambda_l = A_{l+1} P_k
+// + A_l P_{k-1}, P_k = s_k p_k.  Into the m-major complex layout; one thread
+// per (row, map), so that each group's partial sums are read contiguously
+// across the threads.
+__global__ __launch_bounds__(256) void k_adj_finish(LegTables t, int G, int G1,
                                                     const double2 *__restrict__ partial,
                                                     double2 *__restrict__ alm) {
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -585,12 +764,31 @@ __global__ __launch_bounds__(256) void k_adj_finish(LegTables t, int G,
   const int64_t jj = j - t.off[m];
   const int l = m + (int)jj;
   if (l > t.L) return;
-  const double s = t.ascale[j] * (m == 0 ? 1.0 : 2.0);
+  const int64_t rows = t.nlpad * K;
   const int64_t idx = (int64_t)m * (2 * t.L - m + 3) / 2 + jj;
   double2 acc = make_double2(0.0, 0.0);
-  for (int g = 0; g < G; ++g) acc = cadd(acc, partial[(int64_t)g * t.nlpad * K + u]);
+  for (int g = 0; g < G1; ++g) acc = cadd(acc, partial[g * rows + u]);
+  const double s = t.ascale[j];
   acc.x *= s;
-  acc.y = (m == 0) ? 0.0 : acc.y * s;
+  acc.y *= s;
+  if (G1 < G) {
+    double2 pk = make_double2(0.0, 0.0), pp = make_double2(0.0, 0.0);
+    const bool two = !(jj & 1) && jj > 0;
+    for (int g = G1; g < G; ++g) {
+      pk = cadd(pk, partial[g * rows + u]);
+      if (two) pp = cadd(pp, partial[g * rows + u - 2 * K]);
+    }
+    double w = t.pair_w[j / 2], wp = 0.0;
+    if (!(jj & 1)) {
+      w *= sqrt(t.ctil[j + 1]);
+      if (two) wp = t.pair_w[j / 2 - 1] * sqrt(t.ctil[j]);
+    }
+    acc.x += fma(w, pk.x, wp * pp.x);
+    acc.y += fma(w, pk.y, wp * pp.y);
+  }
+  const double cm = m == 0 ? 1.0 : 2.0;
+  acc.x *= cm;
+  acc.y = m == 0 ? 0.0 : acc.y * cm;
   alm[idx * K + k] = acc;
 }
 
@@ -658,6 +856,26 @@ int adjoint_groups_within(const LegTables &t, size_t cap) {
   return G;
 }
 
+// Of G ring groups, those that take the one-step units: their share of the
+// instruction times (above), each unit weighed by sin(theta) (the l > m part of
+// the l, m triangle that its rings reach), at least one; all where the range of
+// the pair form holds no whole unit or there is one group only.
+static int adjoint_one_step_groups(const LegTables &t, int G) {
+  const int ru = adjoint_unit(t);
+  int ua, ub;
+  pair_units(t, ru, &ua, &ub);
+  if (G < 2 || ua >= ub) return G;
+  const int units = (t.R + ru - 1) / ru, kn = std::min(t.K, 4);
+  double one = 0.0, pair = 0.0;
+  for (int c = 0; c < units; ++c) {
+    const double z = ring_z(t.N, std::min(c * ru + ru / 2, t.R - 1)), w = std::sqrt(1.0 - z * z);
+    if (c >= ua && c < ub) pair += w * (2 + 4 * kn);
+    else one += w * (4 + 8 * ((kn + 1) / 2));
+  }
+  const int g1 = (int)std::lround(G * one / (one + pair));
+  return std::max(std::max(1, G - (ub - ua)), std::min(g1, std::min(G - 1, units - (ub - ua))));
+}
+
 hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double *map,
                           double2 *alm, double2 *partial, int G, hipStream_t s) {
   for (int i = 0; i < rt.nlaunch; ++i) {
@@ -717,6 +935,7 @@ hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
+  const int G1 = adjoint_one_step_groups(t, G);
   const unsigned nblk = (unsigned)((t.M + 64) / 64 * 64 * G);
   // passes of up to 4 maps: 8 in one pass leave registers for half the rings
   // only, and with them twice the partial sums to read and write (Nside 1024,
@@ -725,18 +944,21 @@ hipError_t launch_adjoint(const LegTables &t, const RingTables &rt, const double
   for (int kb = 0; kb < t.K; kb += per) {
     const int kn = std::min(per, t.K - kb);
     const bool big = adjoint_unit(t) == 128;
-#define WM_ADJ(CG, GR)                                                                    \
-  hipLaunchKernelGGL((k_legendre_adj<CG, GR>), dim3(nblk), dim3(64), 0, s, t, G, kb, kn, partial)
-    if (kn <= 2 && big) WM_ADJ(1, 8);
-    else if (kn <= 2) WM_ADJ(1, 4);
-    else if (big) WM_ADJ(2, 8);
-    else WM_ADJ(2, 4);
+#define WM_ADJ(KN, GR)                                                                    \
+  hipLaunchKernelGGL((k_legendre_adj<KN, GR>), dim3(nblk), dim3(64), 0, s, t, G, G1, kb,  \
+                     partial)
+    switch (kn) {
+      case 1: if (big) WM_ADJ(1, 8); else WM_ADJ(1, 4); break;
+      case 2: if (big) WM_ADJ(2, 8); else WM_ADJ(2, 4); break;
+      case 3: if (big) WM_ADJ(3, 8); else WM_ADJ(3, 4); break;
+      default: if (big) WM_ADJ(4, 8); else WM_ADJ(4, 4);
+    }
 #undef WM_ADJ
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(k_adj_finish, dim3((unsigned)((t.nlpad * t.K + 255) / 256)), dim3(256), 0,
-                     s, t, G, partial, alm);
+                     s, t, G, G1, partial, alm);
   return hipGetLastError();
 }
 

@@ -164,6 +164,85 @@ __global__ __launch_bounds__(kSegRings) void k_checkpoints(LegTables t) {
   }
 }
 
+// ----------------------------------------------------------- pair form
+//
+// With A_l^2 = (l^2 - m^2) / (4 l^2 - 1), x Lambda_l = A_{l+1} Lambda_{l+1} +
+// A_l Lambda_{l-1}.  Take P_k = Lambda_{l+1} / x at l = m + 2 k.  Then
+//   Lambda_{l+1} = x P_k,   Lambda_l = A_{l+1} P_k + A_l P_{k-1},
+// and, applying the relation twice,
+//   A_{l+2} A_{l+3} P_{k+1} = (x^2 - A_{l+1}^2 - A_{l+2}^2) P_k - A_l A_{l+1} P_{k-1}:
+// one value serves two l.  (K. Ishioka, J. Meteorol. Soc. Japan 96, 2018,
+// computes the transform with such a function.)  Scaled, P_k = s_k p_k with
+// s_{k+1} / s_{k-1} = A_l A_{l+1} / (A_{l+2} A_{l+3}), s_0 = s_1 = 1:
+//   p_{k+1} = (alpha_k y + beta_k) p_k - p_{k-1},
+// two FMAs per two l where the one-step form has four operations.  y is x^2,
+// or x^2 - 1 = -sin^2 theta nearer to the pole, where x^2 itself has lost the
+// angle's low bits; beta_k differs accordingly.
+//
+// The tables, one thread per m: s_k is a product of k ratios, so all of it is
+// computed in double-double and rounded once.
+__device__ __forceinline__ double2 dd_quick(double a, double b) {
+  const double s = a + b;
+  return make_double2(s, b - (s - a));
+}
+__device__ __forceinline__ double2 dd_sum(double a, double b) {
+  const double s = a + b, t = s - a;
+  return make_double2(s, (a - (s - t)) + (b - t));
+}
+__device__ __forceinline__ double2 dd_add(double2 a, double2 b) {
+  const double2 s = dd_sum(a.x, b.x);
+  return dd_quick(s.x, s.y + a.y + b.y);
+}
+__device__ __forceinline__ double2 dd_mul(double2 a, double2 b) {
+  const double p = a.x * b.x;
+  return dd_quick(p, fma(a.x, b.x, -p) + (a.x * b.y + a.y * b.x));
+}
+__device__ __forceinline__ double2 dd_div(double2 a, double2 b) {
+  const double q = a.x / b.x;
+  const double r = fma(-q, b.x, a.x) + (a.y - q * b.y);
+  return dd_quick(q, r / b.x);
+}
+__device__ __forceinline__ double dd_sqrt(double2 a) {
+  const double s = sqrt(a.x);
+  return s + (fma(-s, s, a.x) + a.y) / (2.0 * s);
+}
+// A_l^2; both products are exact
+__device__ __forceinline__ double2 dd_a2(double l, double m) {
+  return dd_div(make_double2((l - m) * (l + m), 0.0),
+                make_double2((2.0 * l - 1.0) * (2.0 * l + 1.0), 0.0));
+}
+
+__global__ __launch_bounds__(64) void k_pair_tables(LegTables t) {
+  const int m = blockIdx.x * 64 + threadIdx.x;
+  if (m > t.M) return;
+  const double dm = (double)m;
+  const int64_t o = t.off[m] / 2;
+  const int n = (t.L - m + kChunk) / kChunk * (kChunk / 2);
+  const double2 one = make_double2(1.0, 0.0);
+  double2 c0 = make_double2(0.0, 0.0), c1 = dd_a2(dm + 1.0, dm);  // A_l^2, A_{l+1}^2
+  double2 tp = one, tk = one;                                     // s_{k-1}^2, s_k^2
+  for (int k = 0; k < n; ++k) {
+    const double l = dm + 2.0 * (double)k;
+    const double2 c2 = dd_a2(l + 2.0, dm), c3 = dd_a2(l + 3.0, dm);
+    const double2 g0 = dd_mul(c0, c1), g1 = dd_mul(c2, c3);
+    const double2 tn = k == 0 ? one : dd_div(dd_mul(tp, g0), g1);
+    const double al = dd_sqrt(dd_div(tk, dd_mul(tn, g1)));
+    const double2 u = dd_add(c1, c2);
+    const double2 v = dd_add(one, make_double2(-u.x, -u.y));
+    t.pair_x[o + k] = make_double2(al, -fma(al, u.x, al * u.y));
+    t.pair_s[o + k] = make_double2(al, fma(al, v.x, al * v.y));
+    t.pair_w[o + k] = dd_sqrt(tk);
+    if (k % (kChunk / 2) == 0)
+      // L~_{l+1} = A_{l+1} Lambda_{l+1} and L~_{l-1} = Lambda_{l-1} / A_l there
+      t.pair_h[(o + k) / (kChunk / 2)] = make_double2(
+          dd_sqrt(dd_div(one, dd_mul(c1, tk))), k == 0 ? 0.0 : dd_sqrt(dd_div(c0, tp)));
+    tp = tk;
+    tk = tn;
+    c0 = c2;
+    c1 = c3;
+  }
+}
+
 // ------------------------------------------------------- a_lm prescale
 
 // map slots of atil: nmaps rounded up to whole blocks of KB
@@ -573,6 +652,11 @@ hipError_t launch_seeds(const LegTables &t, hipStream_t s) {
 
 hipError_t launch_checkpoints(const LegTables &t, hipStream_t s) {
   hipLaunchKernelGGL(k_checkpoints, dim3((unsigned)((t.M + 1) * t.SW)), dim3(kSegRings), 0, s, t);
+  return hipGetLastError();
+}
+
+hipError_t launch_pair_tables(const LegTables &t, hipStream_t s) {
+  hipLaunchKernelGGL(k_pair_tables, dim3(nblocks(t.M + 1, 64)), dim3(64), 0, s, t);
   return hipGetLastError();
 }
 

@@ -83,6 +83,13 @@ bool build_leg_waves(DevArena &a, LegTables &t, int RL, hipStream_t s, int64_t *
 // seeds) and the (l, ring) slots such a sweep executes.
 bool build_leg_segments(DevArena &a, LegTables &t, hipStream_t s, int64_t *T_exec);
 
+// Tables of the pair form of the recurrence and the rings that may use it
+// (t.pair_*), after build_leg_geometry.
+bool build_leg_pairs(DevArena &a, LegTables &t, hipStream_t s);
+
+// z of the 2N northern rings, equator -> pole.
+double ring_z(int N, int r);
+
 // Rings of the long path (kRingLong), in groups of one transform length P
 // (P = h for a power-of-two h, else the Bluestein length): entries
 // vecs[first .. first + count) of (ring pair, hemisphere); with K maps a

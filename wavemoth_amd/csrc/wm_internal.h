@@ -19,6 +19,8 @@ constexpr int kChunk = 16;
 constexpr int kSeedNone = 0x3fffffff;
 // Rings that share their l-segments (LegTables::seg_l0).
 constexpr int kSegRings = 128;
+// Smallest ring unit the pair form is used for (the adjoint's smaller units).
+constexpr int kPairRings = 64;
 // Largest power-of-two FFT length held in LDS by the ring kernels
 // (8192 complex doubles = 128 KiB).
 constexpr int kMaxFFT = 8192;
@@ -55,11 +57,25 @@ struct LegTables {
   int SW = 0;                 // chunks of kSegRings rings
   int *seg_l0 = nullptr;      // [(M+1)*SW] min seed_l over a chunk's rings
   double2 *ckpt = nullptr;    // [(M+1)*3*R] states at the starts of segments 1 .. 3
+  // pair form of the recurrence (k_pair_tables): rings [pair_r0, pair_r1) may
+  // be swept in it; null tables and an empty range when no whole unit lies there
+  int pair_r0 = 0, pair_r1 = 0;
+  double2 *pair_x = nullptr;  // [nlpad/2] (alpha_k, beta_k) for y = x^2
+  double2 *pair_s = nullptr;  // [nlpad/2] (alpha_k, beta_k) for y = x^2 - 1
+  double *pair_w = nullptr;   // [nlpad/2] scale s_k of p_k
+  double2 *pair_h = nullptr;  // [nlpad/kChunk] (L~_{l+1}, L~_{l-1}) -> (p_k, p_{k-1}) / x
   double2 *atil = nullptr;    // [ceil(K/KB)][nlpad][KB] prescaled a_lm (per execute)
   double2 *qbuf = nullptr;    // [R][2][K][M+1] even/odd Legendre sums (q_index)
   int q32 = 0;                // q stored as float2 at the same indices (mixed plans)
   int64_t npix = 0;
 };
+
+// Whole units of `rings` rings that are swept in the pair form: [*a, *b).
+__host__ __device__ inline void pair_units(const LegTables &t, int rings, int *a, int *b) {
+  *a = (t.pair_r0 + rings - 1) / rings;
+  *b = t.pair_r1 / rings;
+  if (*b < *a) *b = *a;
+}
 
 // q(ring pair r, parity p, map k, m) lives at
 //   [r][p][k / G][m][k % G],  G = q_group(K) = min(K, 8),
@@ -286,6 +302,7 @@ hipError_t launch_res_interp(const LegTables &t, const double *img, const ResInt
 hipError_t launch_seeds(const LegTables &t, hipStream_t s);
 hipError_t launch_wave_bounds(const LegTables &t, hipStream_t s);
 hipError_t launch_checkpoints(const LegTables &t, hipStream_t s);
+hipError_t launch_pair_tables(const LegTables &t, hipStream_t s);
 hipError_t launch_prep_alm(const LegTables &t, const double2 *alm, hipStream_t s);
 hipError_t launch_legendre(const LegTables &t, hipStream_t s);
 // Bluestein tables of the lengths hlist[0..nh): chirp[choff + a] =
