@@ -406,8 +406,11 @@ __device__ __forceinline__ double lane_xor4(double x) { return dpp_move<0x1b>(dp
 // even and, times x, the odd sums.  The other units step l by l: 2 vector
 // instructions and, for every 2 maps, one product of which one parity's
 // columns are wanted; per two l and 16 rings 4 + 8 against 2 + 4 instruction
-// times at 1 map, 4 + 16 against 2 + 12 at 3.  A group's units are all of one
-// form: its rows of partial sums are b~_l or the sums of p_k.
+// times at 1 map, 4 + 16 against 2 + 12 at 3 (this kernel with one-step units
+// only / as it is: Nside 2048, lmax 4096, 1 map 6.46 / 4.51 ms; Nside 512, lmax
+// 1024, 3 maps 0.282 / 0.247 ms).  A group's units are all of one form: its
+// rows of partial sums are b~_l or the sums of p_k.
+
 // The units c = c0, c0 + step, ... of `units` one-step units (those below ua,
 // then those from ub on).
 template <int KN, int GR>
@@ -608,14 +611,14 @@ __device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int s
       const int s = t.seed_l[(int64_t)m * t.R + r];
       if (s <= L) seeds[64 * i + lane] = to_pair(t.seed_v[(int64_t)m * t.R + r], t.ring_x[r], s);
     }
-    const bool polar = t.ring_x[c * RU] > 0.7;  // wave-uniform
+    const int zone = __builtin_amdgcn_readfirstlane(pair_zone(t.ring_x[c * RU + RU / 2]));
     double y[GR], prev[GR], cur[GR], bq[KN][GR];
     int sl[GR];
 #pragma unroll
     for (int i = 0; i < GR; ++i) {
       const int r = c * RU + 16 * i + ring;
       const double x = t.ring_x[r];
-      y[i] = polar ? -fma(-x, x, 1.0) : x * x;
+      y[i] = fma(x, x, -pair_centre(zone));
       sl[i] = t.seed_l[(int64_t)m * t.R + r];
       double2 v = make_double2(0.0, 0.0);
       if (u > 0 && cb < nc)
@@ -629,7 +632,7 @@ __device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int s
         bq[k][i] = u >= 2 ? q * x : q;
       }
     }
-    const double2 *pc = (polar ? t.pair_s : t.pair_x) + (offm + l0 - m) / 2;
+    const double2 *pc = t.pair_t + (t.nlpad * zone + offm + l0 - m) / 2;
     double *pr = prow + (int64_t)(l0 - m + (u >> 1)) * rstride + (u & 1);
     unsigned e = KC * (unsigned)(cb < nc ? cb : nc - 1);
     double2 cc[ST];

@@ -155,6 +155,7 @@ Geometry *get_geometry(wavemoth_batch b, int N, int L, int M) {
   g->M = M;
   if (!build_leg_geometry(b->arena, g->base, N, L, M, b->stream, &g->cnt)) return nullptr;
   if (!build_leg_segments(b->arena, g->base, b->stream, &g->T_seg)) return nullptr;
+  if (!build_leg_pairs(b->arena, g->base, b->stream)) return nullptr;
   b->geoms.push_back(std::move(g));
   return b->geoms.back().get();
 }
@@ -278,6 +279,9 @@ bool request_tables(DevArena &keep, DevArena &a, Geometry *g, int K, Shape sh, h
   t.KB = sh.KB;
   const int nkb = (K + sh.KB - 1) / sh.KB;
   if (!dalloc(a, &t.atil, (size_t)t.nlpad * nkb * sh.KB, "batch atil")) return false;
+  if (legendre_pairs(t) &&
+      !dalloc(a, &t.ptil, (size_t)t.nlpad * nkb * sh.KB, "batch pair-form a_lm"))
+    return false;
   if (!dalloc(a, &t.qbuf, (size_t)q_alloc_elems(t.R, K, t.M + 1), "batch qbuf")) return false;
   t.npix = 12 * (int64_t)g->N * g->N;
   *out = t;

@@ -175,12 +175,17 @@ __global__ __launch_bounds__(kSegRings) void k_checkpoints(LegTables t) {
 // computes the transform with such a function.)  Scaled, P_k = s_k p_k with
 // s_{k+1} / s_{k-1} = A_l A_{l+1} / (A_{l+2} A_{l+3}), s_0 = s_1 = 1:
 //   p_{k+1} = (alpha_k y + beta_k) p_k - p_{k-1},
-// two FMAs per two l where the one-step form has four operations.  y is x^2,
-// or x^2 - 1 = -sin^2 theta nearer to the pole, where x^2 itself has lost the
-// angle's low bits; beta_k differs accordingly.
+// two FMAs per two l where the one-step form has four operations.  The rounding
+// of y shifts the angle of all steps alike, so y is x^2 less the middle of its
+// zone of latitude, one rounding of a small number, and beta_k differs by zone.
+// (With y = x^2 or x^2 - 1 the error of E and O is 1.2 .. 1.5 times the one-step
+// form's, with five zones 0.9.)
 //
-// The tables, one thread per m: s_k is a product of k ratios, so all of it is
+// The tables, one wave per m: s_k is a product of k ratios, so all of it is
 // computed in double-double and rounded once.
+// No contraction here: a product fused into one use of it and rounded in
+// another would count its rounding error twice.
+#pragma clang fp contract(off)
 __device__ __forceinline__ double2 dd_quick(double a, double b) {
   const double s = a + b;
   return make_double2(s, b - (s - a));
@@ -202,9 +207,9 @@ __device__ __forceinline__ double2 dd_div(double2 a, double2 b) {
   const double r = fma(-q, b.x, a.x) + (a.y - q * b.y);
   return dd_quick(q, r / b.x);
 }
-__device__ __forceinline__ double dd_sqrt(double2 a) {
+__device__ __forceinline__ double2 dd_sqrt(double2 a) {
   const double s = sqrt(a.x);
-  return s + (fma(-s, s, a.x) + a.y) / (2.0 * s);
+  return dd_quick(s, (fma(-s, s, a.x) + a.y) / (2.0 * s));
 }
 // A_l^2; both products are exact
 __device__ __forceinline__ double2 dd_a2(double l, double m) {
@@ -212,36 +217,65 @@ __device__ __forceinline__ double2 dd_a2(double l, double m) {
                 make_double2((2.0 * l - 1.0) * (2.0 * l + 1.0), 0.0));
 }
 
+// s_{k+1}^2 / s_{k-1}^2 of every second k multiply up; a lane takes a run of k,
+// and the products of the runs before it come by a scan over the wave.
 __global__ __launch_bounds__(64) void k_pair_tables(LegTables t) {
-  const int m = blockIdx.x * 64 + threadIdx.x;
-  if (m > t.M) return;
+  const int m = blockIdx.x, lane = threadIdx.x;
   const double dm = (double)m;
   const int64_t o = t.off[m] / 2;
   const int n = (t.L - m + kChunk) / kChunk * (kChunk / 2);
+  const int len = (n + 127) / 128 * 2;
+  const int ka = lane * len < n ? lane * len : n, ke = ka + len < n ? ka + len : n;
   const double2 one = make_double2(1.0, 0.0);
-  double2 c0 = make_double2(0.0, 0.0), c1 = dd_a2(dm + 1.0, dm);  // A_l^2, A_{l+1}^2
-  double2 tp = one, tk = one;                                     // s_{k-1}^2, s_k^2
-  for (int k = 0; k < n; ++k) {
+  const double la = dm + 2.0 * (double)ka;
+  double2 tp = one, tk = one;  // products of even, of odd k
+  {
+    double2 g0 = dd_mul(dd_a2(la, dm), dd_a2(la + 1.0, dm));
+    for (int k = ka; k < ke; ++k) {
+      const double l = dm + 2.0 * (double)k;
+      const double2 g1 = dd_mul(dd_a2(l + 2.0, dm), dd_a2(l + 3.0, dm));
+      const double2 r = k == 0 ? one : dd_div(g0, g1);
+      if (k & 1) tk = dd_mul(tk, r);
+      else tp = dd_mul(tp, r);
+      g0 = g1;
+    }
+  }
+  for (int d = 1; d <= 32; d *= 2) {
+    const double2 p = make_double2(__shfl_up(tp.x, d), __shfl_up(tp.y, d));
+    const double2 q = make_double2(__shfl_up(tk.x, d), __shfl_up(tk.y, d));
+    if (lane >= d) {
+      tp = dd_mul(tp, p);
+      tk = dd_mul(tk, q);
+    }
+  }
+  tp = make_double2(__shfl_up(tp.x, 1), __shfl_up(tp.y, 1));
+  tk = make_double2(__shfl_up(tk.x, 1), __shfl_up(tk.y, 1));
+  if (lane == 0) tp = tk = one;
+  // tp = s_{k-1}^2, tk = s_k^2
+  double2 c0 = dd_a2(la, dm), c1 = dd_a2(la + 1.0, dm);  // A_l^2, A_{l+1}^2
+  for (int k = ka; k < ke; ++k) {
     const double l = dm + 2.0 * (double)k;
     const double2 c2 = dd_a2(l + 2.0, dm), c3 = dd_a2(l + 3.0, dm);
-    const double2 g0 = dd_mul(c0, c1), g1 = dd_mul(c2, c3);
-    const double2 tn = k == 0 ? one : dd_div(dd_mul(tp, g0), g1);
-    const double al = dd_sqrt(dd_div(tk, dd_mul(tn, g1)));
+    const double2 g1 = dd_mul(c2, c3);
+    const double2 tn = k == 0 ? one : dd_mul(tp, dd_div(dd_mul(c0, c1), g1));
+    const double2 al = dd_sqrt(dd_div(tk, dd_mul(tn, g1)));
     const double2 u = dd_add(c1, c2);
-    const double2 v = dd_add(one, make_double2(-u.x, -u.y));
-    t.pair_x[o + k] = make_double2(al, -fma(al, u.x, al * u.y));
-    t.pair_s[o + k] = make_double2(al, fma(al, v.x, al * v.y));
-    t.pair_w[o + k] = dd_sqrt(tk);
+    for (int z = 0; z < kPairZones; ++z) {
+      const double2 d = dd_add(make_double2(pair_centre(z), 0.0), make_double2(-u.x, -u.y));
+      t.pair_t[t.nlpad / 2 * z + o + k] = make_double2(al.x, dd_mul(al, d).x);
+    }
+    t.pair_w[o + k] = dd_sqrt(tk).x;
     if (k % (kChunk / 2) == 0)
       // L~_{l+1} = A_{l+1} Lambda_{l+1} and L~_{l-1} = Lambda_{l-1} / A_l there
       t.pair_h[(o + k) / (kChunk / 2)] = make_double2(
-          dd_sqrt(dd_div(one, dd_mul(c1, tk))), k == 0 ? 0.0 : dd_sqrt(dd_div(c0, tp)));
+          dd_sqrt(dd_div(one, dd_mul(c1, tk))).x, k == 0 ? 0.0 : dd_sqrt(dd_div(c0, tp)).x);
     tp = tk;
     tk = tn;
     c0 = c2;
     c1 = c3;
   }
 }
+#pragma clang fp contract(fast)
 
 // ------------------------------------------------------- a_lm prescale
 
@@ -267,6 +301,26 @@ __device__ __forceinline__ void prep_entry(const LegTables &t, const double2 *__
   const int kb = kk / KB;
   t.atil[((int64_t)kb * t.nlpad + j) * KB + (kk - kb * KB)] =
       live ? make_double2(a.x * sc, a.y * sc) : make_double2(0.0, 0.0);
+  if (t.ptil) {
+    // the coefficients of p_k in E and of x p_k in O (pair form): s_k (A_{l+1}
+    // a_l + A_{l+2} a_{l+2}) and s_k a_{l+1}, side by side
+    double2 v = make_double2(0.0, 0.0);
+    if (live) {
+      const double w = t.pair_w[j / 2];
+      if (jj & 1) {
+        v = make_double2(w * a.x, w * a.y);
+      } else {
+        const double f = w * sqrt(t.ctil[j + 1]);
+        v = make_double2(f * a.x, f * a.y);
+        if (l + 2 <= L) {  // then the padded range has l + 2
+          const double h = w * sqrt(t.ctil[j + 2]);
+          const double2 b = alm[(idx + 2) * K + kk];
+          v = make_double2(fma(h, b.x, v.x), fma(h, b.y, v.y));
+        }
+      }
+    }
+    t.ptil[((int64_t)kb * t.nlpad + (j - (jj & 1))) * KB + 2 * (kk - kb * KB) + (jj & 1)] = v;
+  }
 }
 
 // The single-plan prescale: one thread per (padded l-entry j, map slot kk),
@@ -297,6 +351,30 @@ template <typename T>
 __device__ __forceinline__ const WM_CONST T *const_view(const T *p) {
   return (const WM_CONST T *)p;
 }
+
+// Brings the coefficient rows of a later chunk into the XCD's L2.  A scalar
+// load that misses it waits for memory, all waves of an m wait with the first
+// one, and the scalar registers hold one step ahead at most: a SIMD's waves
+// together did not have enough arithmetic to cover that (vector units busy 65
+// .. 78 % of the time; one-step sweep at lmax 4096, 1 map without / with this
+// 3.96 / 3.75 ms, lmax 2048 0.576 / 0.541, lmax 1024, 3 maps 0.191 / 0.175).
+// Lane 0 touches the chunk's line of c~_l (or alpha_k, beta_k), lane 1 + i line
+// i of its a~ rows; take() marks where the value has long arrived.
+template <int KB>
+struct RowTouch {
+  const double *p;
+  unsigned stride;  // doubles per chunk
+  double v;
+  __device__ __forceinline__ RowTouch(const double *c, const double *a, int lane) {
+    const int line = lane < 2 * KB ? lane : 2 * KB;
+    p = line == 0 ? c : a + 16 * (line - 1);
+    stride = line == 0 ? kChunk : 2 * KB * kChunk;
+    v = 0.0;
+  }
+  __device__ __forceinline__ void touch(int chunk) { v = p[(unsigned)chunk * stride]; }
+  __device__ __forceinline__ void take() { asm volatile("" ::"v"(v)); }
+};
+constexpr int kTouchAhead = 1;  // chunks: a chunk takes longer than memory; 2 and 4 are no better
 
 // The sweep of up to 3 maps on the vector units: 2 + 2 KB FP64 instructions
 // per (l, ring), their coefficients (c~_l and KB complex a~_l) wave-uniform
@@ -343,7 +421,12 @@ __device__ __forceinline__ void legendre_sweep(
       for (int u = 0; u < 2 * KB; ++u) a[j][u] = at[2 * (int64_t)KB * (l0 + j) + u];
     }
     S = cs[(l0 - m) / kChunk];
+    RowTouch<KB> ahead((const double *)ct + m, (const double *)at + 2 * KB * (int64_t)m, lane);
+    const int lastc = (L - m) / kChunk;
     for (; l0 <= L; l0 += kChunk) {
+      const int far = (l0 - m) / kChunk + kTouchAhead;
+      ahead.take();
+      ahead.touch(far < lastc ? far : lastc);
       if (l0 <= lsmax) {
 #pragma unroll
         for (int i = 0; i < RL; ++i) {
@@ -407,6 +490,124 @@ __device__ __forceinline__ void legendre_sweep(
                 make_double2(acc[i][p][k][0], acc[i][p][k][1]);
       }
     }
+  }
+}
+
+// The same in the pair form: 2 + 4 KB FP64 instructions per two l and ring
+// where the one-step form has 4 + 4 KB, and one move of beta_k for all rings
+// of a lane (a vector instruction reads one scalar operand).  Bound by the
+// vector units: 2.6 ms of 3.4 at lmax 4096, 1 map, where the one-step form
+// takes 3.75; lmax 2048, 2 maps 0.74 / 0.79 ms, lmax 4096, 3 maps 6.6 / 7.2.  pc:
+// (alpha_k, beta_k), at: the KB (E, O) coefficient pairs of p_k.
+template <int RL, int KB>
+__device__ __forceinline__ void legendre_pair_sweep(
+    const LegTables &t, int m, int w, int kbase, int lane, int l0, int lsmax,
+    const WM_CONST double *pc, const WM_CONST double *at, int zone) {
+  constexpr int ST = KB <= 2 ? 2 : 1, KC = kChunk / 2;
+  const int L = t.L, K = t.K;
+  double y[RL], prev[RL], cur[RL];
+  double2 sv[RL];
+  int sl[RL];
+  double acc[RL][2][KB][2];
+#pragma unroll
+  for (int i = 0; i < RL; ++i) {
+    const int r = w * 64 * RL + lane + 64 * i;
+    const double x = t.ring_x[r];
+    y[i] = fma(x, x, -pair_centre(zone));
+    sl[i] = t.seed_l[(int64_t)m * t.R + r];
+    sv[i] = make_double2(0.0, 0.0);
+    if (sl[i] <= L) {
+      // (L~_{l-1}, L~_l) -> (p_{k-1}, p_k)
+      const double2 v = t.seed_v[(int64_t)m * t.R + r];
+      const int64_t j = t.off[m] + sl[i] - m;
+      const double2 h = t.pair_h[j / kChunk];
+      const double rx = 1.0 / x;
+      sv[i] = make_double2(v.x * h.y * rx, fma(x, v.y, -(t.ctil[j] * v.x)) * h.x * rx);
+    }
+    prev[i] = 0.0;
+    cur[i] = 0.0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int k = 0; k < KB; ++k) acc[i][p][k][0] = acc[i][p][k][1] = 0.0;
+  }
+
+  if (l0 <= L) {
+    double al[ST], be[ST], a[ST][4 * KB];
+    const int last = ((L - m) / kChunk + 1) * KC - ST;  // start of the last step
+    int k0 = (l0 - m) / 2;
+#pragma unroll
+    for (int j = 0; j < ST; ++j) {
+      al[j] = pc[2 * (k0 + j)];
+      be[j] = pc[2 * (k0 + j) + 1];
+#pragma unroll
+      for (int u = 0; u < 4 * KB; ++u) a[j][u] = at[4 * (int64_t)KB * (k0 + j) + u];
+    }
+    RowTouch<KB> ahead((const double *)pc, (const double *)at, lane);
+    const int lastc = (L - m) / kChunk;
+    for (; l0 <= L; l0 += kChunk) {
+      const int far = (l0 - m) / kChunk + kTouchAhead;
+      ahead.take();
+      ahead.touch(far < lastc ? far : lastc);
+      if (l0 <= lsmax) {
+#pragma unroll
+        for (int i = 0; i < RL; ++i) {
+          prev[i] = sl[i] == l0 ? sv[i].x : prev[i];
+          cur[i] = sl[i] == l0 ? sv[i].y : cur[i];
+        }
+      }
+#pragma unroll
+      for (int s0 = 0; s0 < KC; s0 += ST) {
+        k0 = k0 < last ? k0 + ST : last;
+        asm volatile("" ::"s"(a[ST - 1][4 * KB - 1]), "s"(al[ST - 1]), "s"(be[ST - 1]));
+        __builtin_amdgcn_sched_barrier(0);
+        double aln[ST], ben[ST], an[ST][4 * KB];
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+          aln[j] = pc[2 * (k0 + j)];
+          ben[j] = pc[2 * (k0 + j) + 1];
+#pragma unroll
+          for (int u = 0; u < 4 * KB; ++u) an[j][u] = at[4 * (int64_t)KB * (k0 + j) + u];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+#pragma unroll
+          for (int i = 0; i < RL; ++i) {
+#pragma unroll
+            for (int k = 0; k < KB; ++k)
+#pragma unroll
+              for (int u = 0; u < 4; ++u)
+                acc[i][u >> 1][k][u & 1] =
+                    fma(cur[i], a[j][4 * k + u], acc[i][u >> 1][k][u & 1]);
+            const double nx = fma(fma(al[j], y[i], be[j]), cur[i], -prev[i]);
+            prev[i] = cur[i];
+            cur[i] = nx;
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+          al[j] = aln[j];
+          be[j] = ben[j];
+#pragma unroll
+          for (int u = 0; u < 4 * KB; ++u) a[j][u] = an[j][u];
+        }
+      }
+    }
+  }
+
+#pragma unroll
+  for (int i = 0; i < RL; ++i) {
+    const int r = w * 64 * RL + lane + 64 * i;
+    const double x = t.ring_x[r];
+#pragma unroll
+    for (int k = 0; k < KB; ++k)
+      if (kbase + k < K) {
+        t.qbuf[q_index(r, 0, kbase + k, m, K, t.M + 1)] =
+            make_double2(acc[i][0][k][0], acc[i][0][k][1]);
+        t.qbuf[q_index(r, 1, kbase + k, m, K, t.M + 1)] =
+            make_double2(x * acc[i][1][k][0], x * acc[i][1][k][1]);
+      }
   }
 }
 
@@ -608,6 +809,16 @@ __device__ __forceinline__ void legendre_item(const LegTables &t, int m, int w, 
   if constexpr (KB <= kMapsVector) {
     const int l0 = __builtin_amdgcn_readfirstlane(t.wstart[(int64_t)m * t.W + w]);
     const int lsmax = __builtin_amdgcn_readfirstlane(t.wseedmax[(int64_t)m * t.W + w]);
+    if (t.ptil && w * 64 * RL >= t.pair_r0 && (w + 1) * 64 * RL <= t.pair_r1) {
+      const int zone =
+          __builtin_amdgcn_readfirstlane(pair_zone(t.ring_x[w * 64 * RL + 32 * RL]));
+      const double2 *pc = t.pair_t + (t.nlpad * zone + offm) / 2;
+      const double2 *pt = t.ptil + ((int64_t)kb * t.nlpad + offm) * KB;
+      legendre_pair_sweep<RL, KB>(t, m, w, kb * KB, lane, l0, lsmax,
+                                  const_view((const double *)pc),
+                                  const_view((const double *)pt), zone);
+      return;
+    }
     legendre_sweep<RL, KB>(t.L, t.R, t.M + 1, t.K, m, w, kb * KB, lane, l0, lsmax,
                            const_view(t.ctil + (offm - m)), const_view(at),
                            const_view(t.cscale + offm / kChunk), t.ring_x, t.seed_l, t.seed_v,
@@ -656,7 +867,7 @@ hipError_t launch_checkpoints(const LegTables &t, hipStream_t s) {
 }
 
 hipError_t launch_pair_tables(const LegTables &t, hipStream_t s) {
-  hipLaunchKernelGGL(k_pair_tables, dim3(nblocks(t.M + 1, 64)), dim3(64), 0, s, t);
+  hipLaunchKernelGGL(k_pair_tables, dim3((unsigned)(t.M + 1)), dim3(64), 0, s, t);
   return hipGetLastError();
 }
 
@@ -694,6 +905,17 @@ int legendre_default_rl(int K, int M, int R) {
   const int KB = legendre_map_block(K, M, R);
   if (!legendre_matrix(KB)) return 2;
   return KB <= 6 && (int64_t)(M + 1) * ((R + 127) / 128) >= 2048 ? 2 : 1;
+}
+// The pair form of 3 maps a pass holds 76 registers, 6 waves a SIMD where the
+// one-step form has 8, so it needs more waves than are resident at once: at
+// 8200 waves (Nside 512, lmax 1024) it takes 0.183 ms where the one-step form
+// takes 0.175, at 32784 (Nside 1024, lmax 2048) and more it is 5 .. 8 % faster.
+// Fewer maps gain at every size (lmax 1024, 1 map 86 / 88 us, 2 maps 126 / 130).
+bool legendre_pairs(const LegTables &t) {
+  int a, b;
+  pair_units(t, 64 * t.RL, &a, &b);
+  return !legendre_matrix(t.KB) && a < b &&
+         (t.KB < 3 || (int64_t)(t.M + 1) * t.W >= 16384);
 }
 int legendre_padded_maps(int K, int KB) {
   return ((K + KB - 1) / KB) * KB;
@@ -804,6 +1026,11 @@ __global__ __launch_bounds__(256) void k_batch_legendre(BatchDev b, int first, i
     t.seg_l0 = tp->seg_l0;
     t.ckpt = tp->ckpt;
     t.atil = tp->atil;
+    t.ptil = tp->ptil;
+    t.pair_r0 = tp->pair_r0;
+    t.pair_r1 = tp->pair_r1;
+    t.pair_t = tp->pair_t;
+    t.pair_h = tp->pair_h;
     t.qbuf = tp->qbuf;
     legendre_item<R_, K_>(t, m, w, kb, lane, seeds[threadIdx.x >> 6]);
   }

@@ -279,8 +279,9 @@ bool build_leg_segments(DevArena &a, LegTables &t, hipStream_t stream, int64_t *
 // Lambda / x in steps of two l: with angle 2 theta per step its two solutions
 // coincide at the equator as well as at the pole, and its sums cancel by x.
 // Error of E and O against 80-bit arithmetic, relative to the one-step form's,
-// by z at lmax 4096: 35 below 0.003, 4.4 below 0.08, 0.8 .. 1.6 between 0.09 and
-// 0.99, 1.8 above; the rings left out near the pole have next to no work.
+// by z at lmax 2048: 39 below 0.006, 3 below 0.09, 1.6 from 1/8 to 0.3, 0.9 .. 1 to
+// 0.7, 0.8 to 0.9, 0.7 to 0.99 (0.9 over all of 1/8 .. 0.99), 1.4 above; the rings
+// left out near the pole have next to no work.
 bool build_leg_pairs(DevArena &a, LegTables &t, hipStream_t stream) {
   int r0 = 0, r1 = t.R;
   while (r0 < t.R && ring_z(t.N, r0) < 0.125) ++r0;
@@ -293,8 +294,7 @@ bool build_leg_pairs(DevArena &a, LegTables &t, hipStream_t stream) {
     t.pair_r0 = t.pair_r1 = 0;
     return true;
   }
-  if (!dalloc(a, &t.pair_x, (size_t)t.nlpad / 2, "pair coefficients")) return false;
-  if (!dalloc(a, &t.pair_s, (size_t)t.nlpad / 2, "pair coefficients")) return false;
+  if (!dalloc(a, &t.pair_t, (size_t)t.nlpad / 2 * kPairZones, "pair coefficients")) return false;
   if (!dalloc(a, &t.pair_w, (size_t)t.nlpad / 2, "pair scales")) return false;
   if (!dalloc(a, &t.pair_h, (size_t)t.nlpad / kChunk, "pair starts")) return false;
   WM_TRY(launch_pair_tables(t, stream), "pair table kernel");
@@ -386,6 +386,10 @@ static bool build_legendre_tables(wavemoth_plan p) {
     }
     if (!dalloc(p->arena, &t.atil, 1, "atil")) return false;
   } else if (!dalloc(p->arena, &t.atil, (size_t)t.nlpad * legendre_padded_maps(p->K, t.KB), "atil")) {
+    return false;
+  } else if (legendre_pairs(t) &&
+             !dalloc(p->arena, &t.ptil, (size_t)t.nlpad * legendre_padded_maps(p->K, t.KB),
+                     "pair-form a_lm")) {
     return false;
   }
   // mixed-precision plans store q in FP32 (float2 elements at the same

@@ -60,11 +60,11 @@ struct LegTables {
   // pair form of the recurrence (k_pair_tables): rings [pair_r0, pair_r1) may
   // be swept in it; null tables and an empty range when no whole unit lies there
   int pair_r0 = 0, pair_r1 = 0;
-  double2 *pair_x = nullptr;  // [nlpad/2] (alpha_k, beta_k) for y = x^2
-  double2 *pair_s = nullptr;  // [nlpad/2] (alpha_k, beta_k) for y = x^2 - 1
+  double2 *pair_t = nullptr;  // [kPairZones][nlpad/2] (alpha_k, beta_k)
   double *pair_w = nullptr;   // [nlpad/2] scale s_k of p_k
   double2 *pair_h = nullptr;  // [nlpad/kChunk] (L~_{l+1}, L~_{l-1}) -> (p_k, p_{k-1}) / x
   double2 *atil = nullptr;    // [ceil(K/KB)][nlpad][KB] prescaled a_lm (per execute)
+  double2 *ptil = nullptr;    // [ceil(K/KB)][nlpad/2][KB][2] a_lm for the pair form, or null
   double2 *qbuf = nullptr;    // [R][2][K][M+1] even/odd Legendre sums (q_index)
   int q32 = 0;                // q stored as float2 at the same indices (mixed plans)
   int64_t npix = 0;
@@ -75,6 +75,17 @@ __host__ __device__ inline void pair_units(const LegTables &t, int rings, int *a
   *a = (t.pair_r0 + rings - 1) / rings;
   *b = t.pair_r1 / rings;
   if (*b < *a) *b = *a;
+}
+
+// Pair form: the zone of a unit whose middle ring has cos(theta) = x, and the
+// centre of the zone's x^2 (1/16, 3/16, 3/8, 5/8, 7/8).
+constexpr int kPairZones = 5;
+__host__ __device__ inline int pair_zone(double x) {
+  const double y = x * x;
+  return y < 0.5 ? (y < 0.125 ? 0 : y < 0.28125 ? 1 : 2) : y < 0.75 ? 3 : 4;
+}
+__host__ __device__ inline double pair_centre(int zone) {
+  return zone < 2 ? (2 * zone + 1) / 16.0 : (2 * zone - 1) / 8.0;
 }
 
 // q(ring pair r, parity p, map k, m) lives at
@@ -303,6 +314,8 @@ hipError_t launch_seeds(const LegTables &t, hipStream_t s);
 hipError_t launch_wave_bounds(const LegTables &t, hipStream_t s);
 hipError_t launch_checkpoints(const LegTables &t, hipStream_t s);
 hipError_t launch_pair_tables(const LegTables &t, hipStream_t s);
+// Whether the sweep of t.KB maps a pass and t.RL rings a lane uses the pair form.
+bool legendre_pairs(const LegTables &t);
 hipError_t launch_prep_alm(const LegTables &t, const double2 *alm, hipStream_t s);
 hipError_t launch_legendre(const LegTables &t, hipStream_t s);
 // Bluestein tables of the lengths hlist[0..nh): chirp[choff + a] =
