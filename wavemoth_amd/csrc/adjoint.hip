@@ -803,12 +803,12 @@ static int adjoint_unit(const LegTables &t) {
 
 int adjoint_groups(const LegTables &t) {
   // one wave per (m, group): groups up to one per unit, while the waves stay
-  // below 40 per SIMD (more only add partial sums to write and read) and the
+  // below 20 per SIMD (more only add partial sums to write and read) and the
   // partial sums below 2 GiB
   const int units = (t.R + adjoint_unit(t) - 1) / adjoint_unit(t);
   const double row_bytes = (double)t.nlpad * t.K * sizeof(double2);
   int G = 1;
-  while (2 * G <= units && (int64_t)(t.M + 1) * 2 * G <= 40960 &&
+  while (2 * G <= units && (int64_t)(t.M + 1) * 2 * G <= 20480 &&
          row_bytes * 2 * G <= 2.0 * 1024 * 1024 * 1024)
     G *= 2;
   return G;
