@@ -407,7 +407,7 @@ __device__ __forceinline__ double lane_xor4(double x) { return dpp_move<0x1b>(dp
 // instructions and, for every 2 maps, one product of which one parity's
 // columns are wanted; per two l and 16 rings 4 + 8 against 2 + 4 instruction
 // times at 1 map, 4 + 16 against 2 + 12 at 3 (this kernel with one-step units
-// only / as it is: Nside 2048, lmax 4096, 1 map 6.46 / 4.51 ms; Nside 512, lmax
+// only / as it is: Nside 2048, lmax 4096, 1 map 6.46 / 4.40 ms; Nside 512, lmax
 // 1024, 3 maps 0.282 / 0.247 ms).  A group's units are all of one form: its
 // rows of partial sums are b~_l or the sums of p_k.
 
@@ -499,9 +499,14 @@ __device__ __forceinline__ void adj_units(const LegTables &t, int c0, int step, 
             cur[i] = v.y;
           }
       }
-      if (3 * ns + j >= nc && cb + j >= nc) {  // past the segment's rows
+      if (3 * ns + j >= nc) {  // past the rows of some segments
+        asm volatile("");  // stays a branch: as selects 4 GR instructions a chunk, 4.51 / 4.40 ms
+        const bool past = cb + j >= nc;
 #pragma unroll
-        for (int i = 0; i < GR; ++i) prev[i] = cur[i] = 0.0;
+        for (int i = 0; i < GR; ++i) {
+          prev[i] = past ? 0.0 : prev[i];
+          cur[i] = past ? 0.0 : cur[i];
+        }
       }
       const unsigned en = kChunk * (unsigned)(cb + j + 1 < nc ? cb + j + 1 : nc - 1);
       double Sn = S;
@@ -665,9 +670,14 @@ __device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int s
             cur[i] = v.y;
           }
       }
-      if (3 * ns + j >= nc && cb + j >= nc) {  // past the segment's rows
+      if (3 * ns + j >= nc) {  // past the rows of some segments
+        asm volatile("");  // stays a branch: as selects 4 GR instructions a chunk, 4.51 / 4.40 ms
+        const bool past = cb + j >= nc;
 #pragma unroll
-        for (int i = 0; i < GR; ++i) prev[i] = cur[i] = 0.0;
+        for (int i = 0; i < GR; ++i) {
+          prev[i] = past ? 0.0 : prev[i];
+          cur[i] = past ? 0.0 : cur[i];
+        }
       }
       const unsigned en = KC * (unsigned)(cb + j + 1 < nc ? cb + j + 1 : nc - 1);
       const int drow = drow0 + KC * j;
