@@ -243,12 +243,13 @@ int64_t wavemoth_plan_info(wavemoth_plan plan, int key);
    their seed and ring tables.  The launches are captured once into a
    HIP graph (unless WAVEMOTH_BATCH_NO_GRAPH) and replayed by every execute.
    With WAVEMOTH_MEASURE the sweep shape of each distinct (Nside, lmax,
-   mmax, nmaps) -- rings per lane and maps per pass -- and the kernel of its
-   wrapping rings (general LDS kernel or register-FFT kernel) are chosen by
-   timing the candidates on the device at plan time (results are kept for
-   the process); otherwise a fixed heuristic chooses, the single plan's.  A
-   measured ring kernel other than the single plan's changes the map in the
-   last bits only.  Executes of one batch must not overlap. */
+   mmax, nmaps) -- its rings per lane, which leave every sum as it is -- and
+   the kernel of its wrapping rings (general LDS kernel or register-FFT
+   kernel) are chosen by timing the candidates on the device at plan time
+   (results are kept for the process); otherwise a fixed heuristic chooses,
+   the single plan's.  A measured ring kernel other than the single plan's
+   changes the map in the last bits only.  Executes of one batch must not
+   overlap. */
 typedef struct _wavemoth_batch *wavemoth_batch;
 #define WAVEMOTH_BATCH_NO_GRAPH 0x200
 

@@ -13,9 +13,9 @@
 // kernels read, so the graph stays valid when the caller's buffers change.
 //
 // Sweep shape per (Nside, lmax, mmax, nmaps): rings per lane RL and maps per
-// pass KB.  Heuristic: KB = nmaps (<= 4) or 8, RL = 2 for nmaps <= 2 else 1.
-// With WAVEMOTH_MEASURE each candidate shape the batched kernel supports is
-// timed on the device and the fastest kept (process-wide wisdom table).
+// pass KB, the single plan's (legendre_map_block, legendre_default_rl).  With
+// WAVEMOTH_MEASURE the RL, which leave every sum the same bits, are timed on
+// the device and the fastest kept (process-wide wisdom table).
 #include <hip/hip_runtime.h>
 
 #include <array>
@@ -63,9 +63,11 @@ int heuristic_rw(int K) { return K >= kRingWideMaps ? 1 : 0; }
 
 std::vector<Shape> candidate_shapes(const Geometry &g, int K) {
   std::vector<Shape> out;
-  const int KB = heuristic_kb(g, K);  // the maps per pass decide the order of the sums
-  for (int RL : {1, 2, 4})
-    if (batch_shape_supported(RL, KB)) out.push_back({RL, KB});
+  LegTables t = g.base;
+  t.KB = heuristic_kb(g, K);  // the maps per pass decide the order of the sums
+  for (int RL : {1, 2, 4})    // the pair form needs a whole ring unit in a wave
+    if (batch_shape_supported(RL, t.KB) && (64 * RL >= kSegRings || !legendre_pairs(t)))
+      out.push_back({RL, t.KB});
   return out;
 }
 
@@ -75,11 +77,18 @@ int64_t nalm_of(int L, int M) {
   return n;
 }
 
+// A wave of two ring units (RL = 4) that differ in the form of their sums takes
+// them in turn: a ring's form may not depend on RL.
 void sweep_items(const LegTables &t, int req, std::vector<BatchLegItem> &out) {
   const int nkb = (t.K + t.KB - 1) / t.KB;
+  std::vector<int> ws;
+  for (int w = 0; w < t.W; ++w) {
+    const bool split = t.RL == 4 && legendre_unit_form(t, 2 * w) != legendre_unit_form(t, 2 * w + 1);
+    ws.push_back(split ? -1 - w : w);
+  }
   for (int m = 0; m <= t.M; ++m)
     for (int kb = 0; kb < nkb; ++kb)
-      for (int w = 0; w < t.W; ++w) out.push_back({req, m, w, kb});
+      for (int w : ws) out.push_back({req, m, w, kb});
 }
 
 // Register-FFT ring class (kind, FFT size P): r16items[first .. first + count)
@@ -463,7 +472,9 @@ bool choose_shape(wavemoth_batch b, Geometry *g, int K, Shape *out, int *measure
     }
   }
   double best = -1.0;
-  for (Shape sh : candidate_shapes(*g, K)) {
+  const std::vector<Shape> shapes = candidate_shapes(*g, K);
+  for (Shape sh : shapes) {
+    if (shapes.size() == 1) break;  // nothing to choose
     const double ms = time_shape(b, g, K, sh);
     if (ms < 0) {
       set_err(std::string("autotuner: timing a sweep shape failed: ") + last_err());

@@ -26,7 +26,7 @@
 // is the GPU form of Ylmgen's firstl and the reference's stripify start
 // rows (wavemoth/lib.pyx:301-368, 397-487); terms skipped before that
 // point are below 1e-32 in magnitude.
-#include "wm_internal.h"
+#include "wm_host.h"
 
 namespace wm {
 
@@ -799,25 +799,29 @@ __device__ __forceinline__ void legendre_sweep_mm(
 }
 
 // One wave's share of the sweep: ring chunk w (rings w*64*RL + lane + 64*i,
-// i < RL) of m, maps kb*KB .. kb*KB+KB-1.  Used by the grid kernel below
-// and by the batched work-queue kernel.
+// i < RL) of m, maps kb*KB .. kb*KB+KB-1; wb: the entry of the wave bounds.
+// Used by the grid kernel below and by the batched work-queue kernel.
 template <int RL, int KB>
 __device__ __forceinline__ void legendre_item(const LegTables &t, int m, int w, int kb,
-                                              int lane, double2 *seeds) {
+                                              int wb, int lane, double2 *seeds) {
   const int64_t offm = t.off[m];
   const double *at = (const double *)(t.atil + ((int64_t)kb * t.nlpad + offm - m) * KB);
   if constexpr (KB <= kMapsVector) {
-    const int l0 = __builtin_amdgcn_readfirstlane(t.wstart[(int64_t)m * t.W + w]);
-    const int lsmax = __builtin_amdgcn_readfirstlane(t.wseedmax[(int64_t)m * t.W + w]);
-    if (t.ptil && w * 64 * RL >= t.pair_r0 && (w + 1) * 64 * RL <= t.pair_r1) {
-      const int zone =
-          __builtin_amdgcn_readfirstlane(pair_zone(t.ring_x[w * 64 * RL + 32 * RL]));
-      const double2 *pc = t.pair_t + (t.nlpad * zone + offm) / 2;
-      const double2 *pt = t.ptil + ((int64_t)kb * t.nlpad + offm) * KB;
-      legendre_pair_sweep<RL, KB>(t, m, w, kb * KB, lane, l0, lsmax,
-                                  const_view((const double *)pc),
-                                  const_view((const double *)pt), zone);
-      return;
+    const int l0 = __builtin_amdgcn_readfirstlane(t.wstart[(int64_t)m * t.W + wb]);
+    const int lsmax = __builtin_amdgcn_readfirstlane(t.wseedmax[(int64_t)m * t.W + wb]);
+    // Form and zone go by the unit of kSegRings rings: a wave of two units has
+    // them in common, or takes its units in turn (sweep_items).
+    if constexpr (64 * RL >= kSegRings) {
+      if (t.ptil && w * 64 * RL >= t.pair_r0 && (w + 1) * 64 * RL <= t.pair_r1) {
+        const int zone =
+            __builtin_amdgcn_readfirstlane(pair_zone(t.ring_x[w * 64 * RL + kSegRings / 2]));
+        const double2 *pc = t.pair_t + (t.nlpad * zone + offm) / 2;
+        const double2 *pt = t.ptil + ((int64_t)kb * t.nlpad + offm) * KB;
+        legendre_pair_sweep<RL, KB>(t, m, w, kb * KB, lane, l0, lsmax,
+                                    const_view((const double *)pc),
+                                    const_view((const double *)pt), zone);
+        return;
+      }
     }
     legendre_sweep<RL, KB>(t.L, t.R, t.M + 1, t.K, m, w, kb * KB, lane, l0, lsmax,
                            const_view(t.ctil + (offm - m)), const_view(at),
@@ -848,7 +852,7 @@ __global__ __launch_bounds__(64) void k_legendre(LegTables t, int nkb, int bpm) 
   const int item = s % bpm;
   const int w = item / nkb, kb = item - w * nkb;
   __shared__ double2 seeds[sweep_lds(RL, KB)];
-  legendre_item<RL, KB>(t, m, w, kb, threadIdx.x, seeds);
+  legendre_item<RL, KB>(t, m, w, kb, w, threadIdx.x, seeds);
 }
 
 // ------------------------------------------------------------ launchers
@@ -911,11 +915,17 @@ int legendre_default_rl(int K, int M, int R) {
 // 8200 waves (Nside 512, lmax 1024) it takes 0.183 ms where the one-step form
 // takes 0.175, at 32784 (Nside 1024, lmax 2048) and more it is 5 .. 8 % faster.
 // Fewer maps gain at every size (lmax 1024, 1 map 86 / 88 us, 2 maps 126 / 130).
+// A ring's sums differ in the last bits between the forms, so the answer goes
+// by the geometry and the map count alone, not by the rings per wave.
 bool legendre_pairs(const LegTables &t) {
   int a, b;
-  pair_units(t, 64 * t.RL, &a, &b);
+  pair_units(t, kSegRings, &a, &b);
   return !legendre_matrix(t.KB) && a < b &&
-         (t.KB < 3 || (int64_t)(t.M + 1) * t.W >= 16384);
+         (t.KB < 3 || (int64_t)(t.M + 1) * ((t.R + kSegRings - 1) / kSegRings) >= 16384);
+}
+int legendre_unit_form(const LegTables &t, int u) {
+  if (!legendre_pairs(t) || u * kSegRings < t.pair_r0 || (u + 1) * kSegRings > t.pair_r1) return -1;
+  return pair_zone(ring_z(t.N, u * kSegRings + kSegRings / 2));
 }
 int legendre_padded_maps(int K, int KB) {
   return ((K + KB - 1) / KB) * KB;
@@ -1032,7 +1042,15 @@ __global__ __launch_bounds__(256) void k_batch_legendre(BatchDev b, int first, i
     t.pair_t = tp->pair_t;
     t.pair_h = tp->pair_h;
     t.qbuf = tp->qbuf;
-    legendre_item<R_, K_>(t, m, w, kb, lane, seeds[threadIdx.x >> 6]);
+    if constexpr (R_ == 4 && K_ <= kMapsVector) {
+      if (w < 0) {  // the wave's two units differ in form
+#pragma unroll 1
+        for (int u = 2 * (-1 - w); u < 2 * -w && u * kSegRings < t.R; ++u)
+          legendre_item<2, K_>(t, m, u, kb, -1 - w, lane, seeds[threadIdx.x >> 6]);
+        continue;
+      }
+    }
+    legendre_item<R_, K_>(t, m, w, kb, w, lane, seeds[threadIdx.x >> 6]);
   }
 }
 

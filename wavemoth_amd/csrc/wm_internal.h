@@ -178,7 +178,7 @@ struct RingTables {
 // sweep and ring stage each run as one persistent work-queue kernel over
 // the union of the requests' work items, in the order the host put them.
 struct BatchLegItem {
-  int req, m, w, kb;  // request, m, ring chunk, map block
+  int req, m, w, kb;  // request, m, ring chunk (w < 0: -1 - w, its ring units in turn), map block
 };
 struct BatchRingItem {
   int req, pair, k;  // request, ring pair, map
@@ -314,8 +314,10 @@ hipError_t launch_seeds(const LegTables &t, hipStream_t s);
 hipError_t launch_wave_bounds(const LegTables &t, hipStream_t s);
 hipError_t launch_checkpoints(const LegTables &t, hipStream_t s);
 hipError_t launch_pair_tables(const LegTables &t, hipStream_t s);
-// Whether the sweep of t.KB maps a pass and t.RL rings a lane uses the pair form.
+// Whether sweeps of t.KB maps a pass use the pair form; the form of its ring
+// unit u (kSegRings rings): the zone of the pair form, -1 the one-step form.
 bool legendre_pairs(const LegTables &t);
+int legendre_unit_form(const LegTables &t, int u);
 hipError_t launch_prep_alm(const LegTables &t, const double2 *alm, hipStream_t s);
 hipError_t launch_legendre(const LegTables &t, hipStream_t s);
 // Bluestein tables of the lengths hlist[0..nh): chirp[choff + a] =
