@@ -776,7 +776,9 @@ static bool run_legendre(wavemoth_plan p, const double2 *d_alm, hipStream_t s) {
   if (p->fly) {
     WM_TRY(launch_seeds(p->lt, s), "seed kernel");
     WM_TRY(launch_wave_bounds(p->lt, s), "wave-bounds kernel");
-    WM_TRY(launch_checkpoints(p->lt, s), "checkpoint kernel");
+    // the matrix-core sweep's; the adjoint has those made with the plan
+    if (p->mix < 0 && !p->res_apply && legendre_matrix(p->lt.KB))
+      WM_TRY(launch_checkpoints(p->lt, s), "checkpoint kernel");
     if (p->mix_ckpt)
       WM_TRY(launch_mix_ckpt(p->lt, p->mix_dtil, p->mix_etil, p->mix_gtil, p->mix_lam_scale,
                              p->mix_ckpt, s),
