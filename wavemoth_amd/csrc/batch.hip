@@ -163,8 +163,6 @@ Geometry *get_geometry(wavemoth_batch b, int N, int L, int M) {
   g->L = L;
   g->M = M;
   if (!build_leg_geometry(b->arena, g->base, N, L, M, b->stream, &g->cnt)) return nullptr;
-  if (!build_leg_segments(b->arena, g->base, b->stream, &g->T_seg)) return nullptr;
-  if (!build_leg_pairs(b->arena, g->base, b->stream)) return nullptr;
   b->geoms.push_back(std::move(g));
   return b->geoms.back().get();
 }
@@ -277,6 +275,24 @@ bool ensure_waves(DevArena &a, Geometry *g, int RL, hipStream_t s) {
   return true;
 }
 
+// The segment or pair-form tables of the geometry into t, if its sweep reads
+// them; built for the first such request.
+bool ensure_sweep_tables(DevArena &a, Geometry *g, LegTables &t, hipStream_t s) {
+  LegTables &b = g->base;
+  if (legendre_matrix(t.KB)) {
+    if (!b.ckpt && !build_leg_segments(a, b, s, &g->T_seg)) return false;
+    t.SW = b.SW;
+    t.seg_l0 = b.seg_l0;
+    t.ckpt = b.ckpt;
+  } else if (legendre_pairs(t)) {
+    if (!b.pair_t && !build_leg_pairs(a, b, s)) return false;
+    t.pair_t = b.pair_t;
+    t.pair_w = b.pair_w;
+    t.pair_h = b.pair_h;
+  }
+  return true;
+}
+
 // Request tables with shape `sh`: the geometry's waves for sh.RL (kept in
 // the batch arena `keep`, since the geometry caches them) plus per-request
 // atil / qbuf allocated in `a`.
@@ -286,6 +302,7 @@ bool request_tables(DevArena &keep, DevArena &a, Geometry *g, int K, Shape sh, h
   LegTables t = g->waves[sh.RL];
   t.K = K;
   t.KB = sh.KB;
+  if (!ensure_sweep_tables(keep, g, t, s)) return false;
   const int nkb = (K + sh.KB - 1) / sh.KB;
   if (!dalloc(a, &t.atil, (size_t)t.nlpad * nkb * sh.KB, "batch atil")) return false;
   if (legendre_pairs(t) &&

@@ -136,6 +136,24 @@ double ring_z(int N, int r) {
   return 4.0 / 3.0 - 2.0 * (double)i / (3.0 * (double)N);
 }
 
+// The pair form takes rings of 1/8 <= z <= 0.99.  Its values are those of
+// Lambda / x in steps of two l: with angle 2 theta per step its two solutions
+// coincide at the equator as well as at the pole, and its sums cancel by x.
+// Error of E and O against 80-bit arithmetic, relative to the one-step form's,
+// by z at lmax 2048: 39 below 0.006, 3 below 0.09, 1.6 from 1/8 to 0.3, 0.9 .. 1 to
+// 0.7, 0.8 to 0.9, 0.7 to 0.99 (0.9 over all of 1/8 .. 0.99), 1.4 above; the rings
+// left out near the pole have next to no work.
+static void set_pair_rings(LegTables &t) {
+  int r0 = 0, r1 = t.R;
+  while (r0 < t.R && ring_z(t.N, r0) < 0.125) ++r0;
+  while (r1 > r0 && ring_z(t.N, r1 - 1) > 0.99) --r1;
+  t.pair_r0 = r0;
+  t.pair_r1 = r1;
+  int ua, ub;
+  pair_units(t, kPairRings, &ua, &ub);
+  if (ua >= ub) t.pair_r0 = t.pair_r1 = 0;
+}
+
 bool build_leg_geometry(DevArena &a, LegTables &t, int N, int L, int M, hipStream_t stream,
                         LegCounts *cnt) {
   const int R = 2 * N;
@@ -144,6 +162,7 @@ bool build_leg_geometry(DevArena &a, LegTables &t, int N, int L, int M, hipStrea
   t.M = M;
   t.K = 0;
   t.R = R;
+  set_pair_rings(t);
 
   std::vector<int64_t> off(M + 1);
   int64_t tot = 0;
@@ -275,25 +294,8 @@ bool build_leg_segments(DevArena &a, LegTables &t, hipStream_t stream, int64_t *
   return true;
 }
 
-// The pair form takes rings of 1/8 <= z <= 0.99.  Its values are those of
-// Lambda / x in steps of two l: with angle 2 theta per step its two solutions
-// coincide at the equator as well as at the pole, and its sums cancel by x.
-// Error of E and O against 80-bit arithmetic, relative to the one-step form's,
-// by z at lmax 2048: 39 below 0.006, 3 below 0.09, 1.6 from 1/8 to 0.3, 0.9 .. 1 to
-// 0.7, 0.8 to 0.9, 0.7 to 0.99 (0.9 over all of 1/8 .. 0.99), 1.4 above; the rings
-// left out near the pole have next to no work.
 bool build_leg_pairs(DevArena &a, LegTables &t, hipStream_t stream) {
-  int r0 = 0, r1 = t.R;
-  while (r0 < t.R && ring_z(t.N, r0) < 0.125) ++r0;
-  while (r1 > r0 && ring_z(t.N, r1 - 1) > 0.99) --r1;
-  t.pair_r0 = r0;
-  t.pair_r1 = r1;
-  int ua, ub;
-  pair_units(t, kPairRings, &ua, &ub);
-  if (ua >= ub) {
-    t.pair_r0 = t.pair_r1 = 0;
-    return true;
-  }
+  if (t.pair_r0 == t.pair_r1) return true;
   if (!dalloc(a, &t.pair_t, (size_t)t.nlpad / 2 * kPairZones, "pair coefficients")) return false;
   if (!dalloc(a, &t.pair_w, (size_t)t.nlpad / 2, "pair scales")) return false;
   if (!dalloc(a, &t.pair_h, (size_t)t.nlpad / kChunk, "pair starts")) return false;
@@ -304,18 +306,31 @@ bool build_leg_pairs(DevArena &a, LegTables &t, hipStream_t stream) {
 
 }  // namespace wm
 
+// Whether the plan's synthesis runs the FP64 sweep (legendre.hip).
+static bool fp64_sweep(wavemoth_plan p) { return p->mix < 0 && !p->res_apply; }
+
+// The segment and pair-form tables, which at one map take as much memory as
+// the other tables and q together (Nside 2048, lmax 4096: 805 and 378 MB): for
+// the adjoint, which may not allocate them when called, and for the sweeps that
+// read them.
+static bool build_sweep_tables(wavemoth_plan p) {
+  LegTables &t = p->lt;
+  const bool matrix = fp64_sweep(p) && legendre_matrix(t.KB);
+  int64_t T_seg = 0;
+  if ((p->rt.adj_ok || matrix) && !build_leg_segments(p->arena, t, p->stream, &T_seg)) return false;
+  if (matrix) p->T_exec = T_seg;
+  return !(p->rt.adj_ok || (fp64_sweep(p) && legendre_pairs(t))) ||
+         build_leg_pairs(p->arena, t, p->stream);
+}
+
 static bool build_legendre_tables(wavemoth_plan p) {
   LegTables &t = p->lt;
   if (!build_leg_geometry(p->arena, t, p->N, p->L, p->M, p->stream, &p->cnt)) return false;
   int RL = p->rl_choice > 0 ? p->rl_choice : legendre_default_rl(p->K, t.M, t.R);
   if (p->mix >= 0) RL = mix_rings_per_lane_table();  // one wave-table entry per workgroup
-  int64_t T_seg = 0;
-  if (!build_leg_segments(p->arena, t, p->stream, &T_seg)) return false;
-  if (!build_leg_pairs(p->arena, t, p->stream)) return false;
   if (!build_leg_waves(p->arena, t, RL, p->stream, &p->T_exec)) return false;
   t.K = p->K;
   t.KB = legendre_map_block(p->K, t.M, t.R);
-  if (p->mix < 0 && legendre_matrix(t.KB)) p->T_exec = T_seg;
   if (p->mix >= 0) {
     // the mixed path reads the pre-split B operand instead of atil
     const int cpb = mix_cols_per_block();
@@ -387,7 +402,7 @@ static bool build_legendre_tables(wavemoth_plan p) {
     if (!dalloc(p->arena, &t.atil, 1, "atil")) return false;
   } else if (!dalloc(p->arena, &t.atil, (size_t)t.nlpad * legendre_padded_maps(p->K, t.KB), "atil")) {
     return false;
-  } else if (legendre_pairs(t) &&
+  } else if (fp64_sweep(p) && legendre_pairs(t) &&
              !dalloc(p->arena, &t.ptil, (size_t)t.nlpad * legendre_padded_maps(p->K, t.KB),
                      "pair-form a_lm")) {
     return false;
@@ -777,7 +792,7 @@ static bool run_legendre(wavemoth_plan p, const double2 *d_alm, hipStream_t s) {
     WM_TRY(launch_seeds(p->lt, s), "seed kernel");
     WM_TRY(launch_wave_bounds(p->lt, s), "wave-bounds kernel");
     // the matrix-core sweep's; the adjoint has those made with the plan
-    if (p->mix < 0 && !p->res_apply && legendre_matrix(p->lt.KB))
+    if (fp64_sweep(p) && legendre_matrix(p->lt.KB))
       WM_TRY(launch_checkpoints(p->lt, s), "checkpoint kernel");
     if (p->mix_ckpt)
       WM_TRY(launch_mix_ckpt(p->lt, p->mix_dtil, p->mix_etil, p->mix_gtil, p->mix_lam_scale,
@@ -1088,7 +1103,8 @@ wavemoth_plan wavemoth_plan_to_healpix(int Nside, int lmax, int mmax, int nmaps,
     delete p;
     return nullptr;
   }
-  if (!build_legendre_tables(p) || !build_ring_tables(p) || !build_resource_apply(p)) {
+  if (!build_legendre_tables(p) || !build_ring_tables(p) || !build_sweep_tables(p) ||
+      !build_resource_apply(p)) {
     std::string e = g_err;
     free_plan(p);
     g_err = e;

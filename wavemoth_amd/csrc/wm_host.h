@@ -83,8 +83,8 @@ bool build_leg_waves(DevArena &a, LegTables &t, int RL, hipStream_t s, int64_t *
 // seeds) and the (l, ring) slots such a sweep executes.
 bool build_leg_segments(DevArena &a, LegTables &t, hipStream_t s, int64_t *T_exec);
 
-// Tables of the pair form of the recurrence and the rings that may use it
-// (t.pair_*), after build_leg_geometry.
+// Tables of the pair form of the recurrence (t.pair_t, t.pair_w, t.pair_h)
+// where rings may use it (t.pair_r0, t.pair_r1, from build_leg_geometry).
 bool build_leg_pairs(DevArena &a, LegTables &t, hipStream_t s);
 
 // z of the 2N northern rings, equator -> pole.

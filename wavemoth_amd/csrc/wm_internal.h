@@ -57,8 +57,8 @@ struct LegTables {
   int SW = 0;                 // chunks of kSegRings rings
   int *seg_l0 = nullptr;      // [(M+1)*SW] min seed_l over a chunk's rings
   double2 *ckpt = nullptr;    // [(M+1)*3*R] states at the starts of segments 1 .. 3
-  // pair form of the recurrence (k_pair_tables): rings [pair_r0, pair_r1) may
-  // be swept in it; null tables and an empty range when no whole unit lies there
+  // pair form of the recurrence (k_pair_tables, null without it): rings
+  // [pair_r0, pair_r1) may be swept in it, an empty range when they hold no unit
   int pair_r0 = 0, pair_r1 = 0;
   double2 *pair_t = nullptr;  // [kPairZones][nlpad/2] (alpha_k, beta_k)
   double *pair_w = nullptr;   // [nlpad/2] scale s_k of p_k
