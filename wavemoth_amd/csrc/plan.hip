@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -95,13 +96,50 @@ struct _wavemoth_plan {
   int32_t *res_codes = nullptr;
   std::vector<int> res_depth_op;
   std::vector<int64_t> res_depth_item;
-  // streams of the host-buffer copies' helper threads, made on first use
-  std::vector<hipStream_t> side;
+  const hipStream_t *side = nullptr;  // side_streams(device), from the first large host copy on
   // stage timing (extension): events recorded around prep / sweep / rings
   bool profiling = false;
   std::vector<hipEvent_t> ev_free;
   std::vector<std::array<hipEvent_t, 4>> ev_used;
 };
+
+// The streams of the host-buffer copies' helper threads: one set per device
+// for all plans that copy (users: +1 takes it, -1 gives it back), destroyed with
+// the last of them.  A new stream and its first pageable copy cost 1.5 ms, up to
+// 8 where they get a hardware queue, and 4 MB of pinned memory, so a plan has
+// none of its own (first calls of further plans, Nside 128, 8 maps: 2.5 ms with
+// own streams, 1.6 with these, 2.4 in one copy; calls after it 0.6 .. 0.9, 0.95
+// in one copy).  Copies of several threads may share a stream: each waits for
+// all it holds.  nullptr if they cannot be made.
+constexpr int kCopyParts = 4;
+static const hipStream_t *side_streams(int device, int users) {
+  struct Set {
+    int users = 0;
+    hipStream_t s[kCopyParts - 1] = {};
+  };
+  constexpr int kMaxDevices = 64;
+  static std::mutex mu;
+  static Set sets[kMaxDevices];
+  if (device < 0 || device >= kMaxDevices) return nullptr;
+  std::lock_guard<std::mutex> lock(mu);
+  Set &set = sets[device];
+  bool ok = true;
+  if (set.users == 0 && users > 0) {
+    int cur = device;
+    ok = hipGetDevice(&cur) == hipSuccess && hipSetDevice(device) == hipSuccess;
+    for (hipStream_t &s : set.s)
+      ok = ok && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess;
+    (void)hipSetDevice(cur);
+    if (!ok) (void)hipGetLastError();
+  }
+  if (ok) set.users += users;
+  if (set.users == 0)
+    for (hipStream_t &s : set.s) {
+      if (s) (void)hipStreamDestroy(s);
+      s = nullptr;
+    }
+  return ok ? set.s : nullptr;
+}
 
 static void release_events(wavemoth_plan p) {
   for (auto &a : p->ev_used)
@@ -115,7 +153,7 @@ static void free_plan(wavemoth_plan p) {
   release_events(p);
   for (hipEvent_t e : p->ev_free) (void)hipEventDestroy(e);
   p->arena.release();
-  for (hipStream_t s : p->side) (void)hipStreamDestroy(s);
+  if (p->side) side_streams(p->device, -1);
   if (p->stream) (void)hipStreamDestroy(p->stream);
   delete p;
 }
@@ -1130,19 +1168,17 @@ static bool ensure_staging(wavemoth_plan p) {
 // stream.  Large ones are cut into four parts, each copied by a thread on a
 // stream of its own: pageable memory goes through the runtime's bounce buffers
 // with one memcpy thread per call, which is what limits it (100 MB down: one
-// thread 5.7 ms, two 3.3, four 2.5, eight 2.5; the link takes 1.8).
+// thread 5.7 ms, two 3.3, four 2.5, eight 2.5; the link takes 1.8).  Repeated
+// calls on the same arrays, medians of three processes, one copy / four parts:
+// Nside 256, 1 map 0.53 / 0.35 ms, 1024 7.9 / 4.2, 2048 33 / 16; on arrays new to
+// the process the first touch of their pages adds to both.
 constexpr size_t kCopySplit = (size_t)2 << 20;
-constexpr int kCopyParts = 4;
 static bool copy_host(wavemoth_plan p, void *dst, const void *src, size_t bytes,
                       hipMemcpyKind kind, const char *what) {
-  if (bytes < kCopySplit) {
+  if (bytes >= kCopySplit && !p->side) p->side = side_streams(p->device, 1);
+  if (bytes < kCopySplit || !p->side) {
     WM_TRY(hipMemcpyAsync(dst, src, bytes, kind, p->stream), what);
     return true;
-  }
-  while ((int)p->side.size() < kCopyParts - 1) {
-    hipStream_t s = nullptr;
-    WM_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), what);
-    p->side.push_back(s);
   }
   WM_TRY(hipStreamSynchronize(p->stream), what);  // the buffers are not in use
   const size_t part = bytes / kCopyParts / 4096 * 4096;
