@@ -982,11 +982,13 @@ __global__ __launch_bounds__(256) void k_batch_prep(BatchDev b) {
   prep_entry(t, b.alm[lo], j, (int)(u - j * Kp), t.KB);
 }
 
-// (RL, KB) shapes of the sweep
-#define WM_SWEEP_SHAPES(X)                                                    \
-  X(1, 1) X(1, 2) X(1, 3) X(2, 1) X(2, 2) X(2, 3) X(4, 1) X(4, 2) X(4, 3)     \
-  X(1, 4) X(2, 4) X(1, 6) X(2, 6) X(1, 8) X(2, 8)                             \
+// (RL, KB) shapes of the single-plan sweep (those of legendre_default_rl and
+// legendre_map_block) and the further ones of a measured batch
+#define WM_PLAN_SHAPES(X)                                                     \
+  X(2, 1) X(2, 2) X(2, 3) X(1, 4) X(2, 4) X(1, 6) X(2, 6) X(1, 8)             \
   X(1, 10) X(1, 12) X(1, 14) X(1, 16)
+#define WM_SWEEP_SHAPES(X)                                                    \
+  WM_PLAN_SHAPES(X) X(1, 1) X(1, 2) X(1, 3) X(4, 1) X(4, 2) X(4, 3) X(2, 8)
 
 bool batch_shape_supported(int RL, int KB) { return batch_shape_index(RL, KB) >= 0; }
 
@@ -1092,7 +1094,7 @@ hipError_t launch_batch_legendre(const BatchDev &b, int RL, int KB, int first, i
 hipError_t launch_legendre(const LegTables &t, hipStream_t s) {
 #define WM_LAUNCH(R_, K_) \
   if (t.RL == R_ && t.KB == K_) return launch_leg_t<R_, K_>(t, s);
-  WM_SWEEP_SHAPES(WM_LAUNCH)
+  WM_PLAN_SHAPES(WM_LAUNCH)
 #undef WM_LAUNCH
   return hipErrorInvalidValue;
 }

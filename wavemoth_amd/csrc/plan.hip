@@ -53,7 +53,6 @@ struct _wavemoth_plan {
   double *d_map = nullptr;
   bool phase_shifts = true;
   bool fly = false;
-  int rl_choice = 0;  // rings per lane of the Legendre sweep (0 = heuristic)
   // mixed-precision contraction (extension): -1 = FP64 sweep, else scheme
   // 0 FP32 MFMA, 1 BF16x3, 2 BF16x6
   int mix = -1;
@@ -364,7 +363,7 @@ static bool build_sweep_tables(wavemoth_plan p) {
 static bool build_legendre_tables(wavemoth_plan p) {
   LegTables &t = p->lt;
   if (!build_leg_geometry(p->arena, t, p->N, p->L, p->M, p->stream, &p->cnt)) return false;
-  int RL = p->rl_choice > 0 ? p->rl_choice : legendre_default_rl(p->K, t.M, t.R);
+  int RL = legendre_default_rl(p->K, t.M, t.R);
   if (p->mix >= 0) RL = mix_rings_per_lane_table();  // one wave-table entry per workgroup
   if (!build_leg_waves(p->arena, t, RL, p->stream, &p->T_exec)) return false;
   t.K = p->K;
