@@ -424,7 +424,7 @@ __device__ __forceinline__ void adj_units(const LegTables &t, int c0, int step, 
   const int64_t offm = t.off[m];
   const double *ct0 = t.ctil + (offm - m);
   const double *cs0 = t.cscale + offm / kChunk;
-  const unsigned rstride = 2 * (unsigned)K;  // doubles per l row of the partial sums
+  const int64_t rstride = 2 * (int64_t)K;  // doubles per l row of the partial sums
   bool first = true;
   for (int ci = c0; ci < units; ci += step) {
     const int c = ci < ua ? ci : ci - ua + ub;
@@ -481,7 +481,7 @@ __device__ __forceinline__ void adj_units(const LegTables &t, int c0, int step, 
                        blk < ns * (kChunk / ST);
 #pragma unroll
       for (int cg = 0; cg < CG; ++cg)
-        o[cg] = rok && 4 * cg + u < 2 * kn ? pr[(unsigned)dr * rstride + 4 * cg] : 0.0;
+        o[cg] = rok && 4 * cg + u < 2 * kn ? pr[dr * rstride + 4 * cg] : 0.0;
     };
     wave_sync_lds();
     load_old(0, old);
@@ -519,7 +519,7 @@ __device__ __forceinline__ void adj_units(const LegTables &t, int c0, int step, 
         for (int s = 0; s < ST; ++s) cn[s] = ct[(s0 + ST < kChunk ? e + s0 + ST : en) + s];
         if (s0 + ST == kChunk) Sn = cs[en / kChunk];
         const bool rok = dok && l0 + drow + s0 <= L;
-        const unsigned ro = (unsigned)(drow + s0) * rstride;
+        const int64_t ro = (drow + s0) * rstride;
         load_old(j * (kChunk / ST) + s0 / ST + 1, on);
         __builtin_amdgcn_sched_barrier(0);
         double d[ST][CG];
@@ -590,7 +590,7 @@ __device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int s
   const int64_t offm = t.off[m];
   const double *ct0 = t.ctil + (offm - m);
   const double2 *h0 = t.pair_h + offm / kChunk;
-  const unsigned rstride = 2 * (unsigned)K;  // doubles per l row of the partial sums
+  const int64_t rstride = 2 * (int64_t)K;  // doubles per l row of the partial sums
   bool first = true;
   for (int c = c0; c < ub; c += step) {
     const int l0 = __builtin_amdgcn_readfirstlane(
@@ -652,7 +652,7 @@ __device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int s
       const bool rok = !first && ds * ns + blk / (KC / ST) < nc && l0 + 2 * dr <= L &&
                        blk < ns * (KC / ST);
 #pragma unroll
-      for (int k = 0; k < KN; ++k) o[k] = rok ? pr[2 * (unsigned)dr * rstride + 2 * k] : 0.0;
+      for (int k = 0; k < KN; ++k) o[k] = rok ? pr[2 * dr * rstride + 2 * k] : 0.0;
     };
     wave_sync_lds();
     load_old(0, old);
@@ -689,7 +689,7 @@ __device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int s
 #pragma unroll
         for (int s = 0; s < ST; ++s) cn[s] = pc[(s0 + ST < KC ? e + s0 + ST : en) + s];
         const bool rok = dok && l0 + 2 * (drow + s0) <= L;
-        const unsigned ro = 2 * (unsigned)(drow + s0) * rstride;
+        const int64_t ro = 2 * (drow + s0) * rstride;
         load_old(j * (KC / ST) + s0 / ST + 1, on);
         __builtin_amdgcn_sched_barrier(0);
         double d[ST][KN];

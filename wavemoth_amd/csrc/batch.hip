@@ -57,8 +57,8 @@ struct Shape {
 std::mutex g_wisdom_mu;
 std::map<std::tuple<int, int, int, int>, Shape> g_wisdom;  // (N, L, M, K) -> shape
 
-int heuristic_kb(const Geometry &g, int K) { return legendre_map_block(K, g.M, 2 * g.N); }
-int heuristic_rl(const Geometry &g, int K) { return legendre_default_rl(K, g.M, 2 * g.N); }
+int heuristic_kb(const Geometry &g, int K) { return legendre_map_block(K, g.L, g.M, 2 * g.N); }
+int heuristic_rl(const Geometry &g, int K) { return legendre_default_rl(K, g.L, g.M, 2 * g.N); }
 int heuristic_rw(int K) { return K >= kRingWideMaps ? 1 : 0; }
 
 std::vector<Shape> candidate_shapes(const Geometry &g, int K) {

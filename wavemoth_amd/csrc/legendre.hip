@@ -892,12 +892,14 @@ hipError_t launch_wave_bounds(const LegTables &t, hipStream_t s) {
 // Waves of the vector form at which the two are even: 3 maps between 3072
 // (Nside 256, lmax 767: 114 / 79 us) and 8200 (Nside 512: 207 / 250 us),
 // fewer maps between 514 (Nside 128: 23 / 17 us) and 2052 (Nside 256: 44 / 45).
-int legendre_map_block(int K, int M, int R) {
+int legendre_map_block(int K, int L, int M, int R) {
   if (K <= kMapsVector) {
     const int64_t waves = (int64_t)(M + 1) * ((R + 127) / 128);
     return waves < (K < 3 ? 1024 : 6144) ? kMapsVector + 1 : K;
   }
-  const int passes = (K + 15) / 16, kb = (K + passes - 1) / passes;
+  // the matrix form's row offsets are 32 bits: 2 KB (lmax + kChunk) below 2^32
+  const int most = L < (1 << 27) - kChunk ? 16 : 6;
+  const int passes = (K + most - 1) / most, kb = (K + passes - 1) / passes;
   return (kb + 1) / 2 * 2;
 }
 bool legendre_matrix(int KB) { return KB > kMapsVector; }
@@ -905,8 +907,8 @@ bool legendre_matrix(int KB) { return KB > kMapsVector; }
 // serves twice the rings; one: 0.87 ms where two take 0.60), two on the matrix
 // cores while the accumulators leave two waves per SIMD and the waves fill
 // the chip (6 maps: 1.87 ms, with one 2.01; 8 maps: 2.08, with one 2.02).
-int legendre_default_rl(int K, int M, int R) {
-  const int KB = legendre_map_block(K, M, R);
+int legendre_default_rl(int K, int L, int M, int R) {
+  const int KB = legendre_map_block(K, L, M, R);
   if (!legendre_matrix(KB)) return 2;
   return KB <= 6 && (int64_t)(M + 1) * ((R + 127) / 128) >= 2048 ? 2 : 1;
 }

@@ -363,11 +363,11 @@ static bool build_sweep_tables(wavemoth_plan p) {
 static bool build_legendre_tables(wavemoth_plan p) {
   LegTables &t = p->lt;
   if (!build_leg_geometry(p->arena, t, p->N, p->L, p->M, p->stream, &p->cnt)) return false;
-  int RL = legendre_default_rl(p->K, t.M, t.R);
+  int RL = legendre_default_rl(p->K, t.L, t.M, t.R);
   if (p->mix >= 0) RL = mix_rings_per_lane_table();  // one wave-table entry per workgroup
   if (!build_leg_waves(p->arena, t, RL, p->stream, &p->T_exec)) return false;
   t.K = p->K;
-  t.KB = legendre_map_block(p->K, t.M, t.R);
+  t.KB = legendre_map_block(p->K, t.L, t.M, t.R);
   if (p->mix >= 0) {
     // the mixed path reads the pre-split B operand instead of atil
     const int cpb = mix_cols_per_block();

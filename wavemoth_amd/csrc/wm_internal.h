@@ -263,8 +263,8 @@ hipError_t launch_mixr(const LegTables &t, const void *bmat, int NCp, int64_t pa
 
 // Shape of the Legendre sweep for nmaps = K on a geometry: maps per pass KB,
 // rings per wave / 64; whether the passes run on the matrix cores; map slots.
-int legendre_map_block(int K, int M, int R);
-int legendre_default_rl(int K, int M, int R);
+int legendre_map_block(int K, int L, int M, int R);
+int legendre_default_rl(int K, int L, int M, int R);
 bool legendre_matrix(int KB);
 int legendre_padded_maps(int K, int KB);
 
