@@ -424,7 +424,7 @@ __device__ __forceinline__ void adj_units(const LegTables &t, int c0, int step, 
   const int64_t offm = t.off[m];
   const double *ct0 = t.ctil + (offm - m);
   const double *cs0 = t.cscale + offm / kChunk;
-  const int64_t rstride = 2 * (int64_t)K;  // doubles per l row of the partial sums
+  const int64_t rstride = 2 * (int64_t)K;  // doubles per row of the partial sums (times lmax past 2^32)
   bool first = true;
   for (int ci = c0; ci < units; ci += step) {
     const int c = ci < ua ? ci : ci - ua + ub;
@@ -590,7 +590,7 @@ __device__ __forceinline__ void adj_pair_units(const LegTables &t, int c0, int s
   const int64_t offm = t.off[m];
   const double *ct0 = t.ctil + (offm - m);
   const double2 *h0 = t.pair_h + offm / kChunk;
-  const int64_t rstride = 2 * (int64_t)K;  // doubles per l row of the partial sums
+  const int64_t rstride = 2 * (int64_t)K;  // doubles per row of the partial sums (times lmax past 2^32)
   bool first = true;
   for (int c = c0; c < ub; c += step) {
     const int l0 = __builtin_amdgcn_readfirstlane(
@@ -872,7 +872,10 @@ int adjoint_groups_within(const LegTables &t, size_t cap) {
 // Of G ring groups, those that take the one-step units: their share of the
 // instruction times (above), each unit weighed by sin(theta) (the l > m part of
 // the l, m triangle that its rings reach), at least one; all where the range of
-// the pair form holds no whole unit or there is one group only.
+// the pair form holds no whole unit or there is one group only.  A pass of 4
+// maps is what is priced: the actual passes (3 maps at 5, 6 and 9) give no better
+// split (5 .. 9 maps within 2 %; Nside 300, lmax 899: 13 maps 1.42 ms so, 1.53
+// with the actual ones).
 static int adjoint_one_step_groups(const LegTables &t, int G) {
   const int ru = adjoint_unit(t);
   int ua, ub;
